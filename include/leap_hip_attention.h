@@ -358,7 +358,10 @@ int leap_hip_attention_block_views_get(leap_hip_attention *h, leap_hip_attention
  * sequence) with the same loads and only sums them (the launch plus
  * bare-stream floor).  pos is device memory as in step_batched_async, or
  * NULL for every sequence at max_pos.  Neither kind writes memory or
- * changes the cache.  n_seq = 1, pos = NULL, max_pos = the position,
+ * changes the cache.  For a batch that the step cuts into equal runs over
+ * its sequences (lengths or a count that do not cut evenly over the compute
+ * units), the floors run the uniform chunks it would otherwise have.
+ * n_seq = 1, pos = NULL, max_pos = the position,
  * total_rows = position + 1 is the single-sequence step.  Kind 3, for a
  * layer with weights set (one sequence, pos NULL, total_rows = max_pos +
  * 1): the floor of leap_hip_attention_block_async, three launches with the

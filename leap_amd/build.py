@@ -54,7 +54,7 @@ def _run(cmd):
 
 
 HIP_SOURCES = ("leap_hip_attention", "kernels_decode", "kernels_decode_64", "kernels_decode_64p",
-               "kernels_decode_128", "kernels_decode_128p", "kernels_gemv", "kernels_q8")
+               "kernels_decode_128", "kernels_decode_128p", "kernels_decode_64f", "kernels_decode_128f", "kernels_gemv", "kernels_q8")
 
 
 def _hip_objects(build_dir: str, defines=()):

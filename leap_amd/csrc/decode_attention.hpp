@@ -101,6 +101,66 @@ __host__ __device__ constexpr int counters_per_group(int grid_chunks)
     return (1 + (grid_chunks + kSubGroup - 1) / kSubGroup) * kCtrStride;
 }
 
+// ---- flat launches (decode_attention_flat_kernel) ----------------------------
+//
+// A batch's groups (sequence, KV head) rarely cut into equal chunks that are
+// a whole number per CU: lengths differ, and the sequences need not divide
+// the CUs.  A flat launch has n_wg workgroups per XCD, all resident, and cuts
+// the XCD's rows, its groups ("items": item i of XCD x is group 8 i + x) laid
+// end to end, into n_wg runs of equal length.  A run that reaches over an
+// item's end is two segments or more, each a chunk of its item.  Starting a
+// segment costs a workgroup about as much as kFlatSegmentRows rows (its q,
+// first rows, combine and merge lie in series), so an item counts that many
+// rows more than it has, ahead of its first: a run that holds a start takes
+// fewer rows.
+// Measured against 0, 32, 64, 96, 192 and 256 rows over ragged batches of
+// 2-64 sequences of 550-4400 rows at the shapes of Llama-3-8B, Llama-3-70B
+// and TinyLlama: 128 is the fastest or within 2% in the mean (0: +5-8%).
+constexpr int kFlatSegmentRows = 128;
+constexpr int kFlatMinRun = 64;          // rows of a run at least: one pass of 4 waves
+constexpr int kFlatMaxItems = 64;        // items per XCD at most: one lane each
+// A run of a large batch holds thousands of rows.  Every kFlatFlushPasses
+// passes a wave adds its output accumulators to sums in LDS and starts them
+// anew, so that no fp32 sum is longer than a uniform chunk's.  Error against
+// 64 bits, 64 sequences of 512-8192 rows of Llama-3-8B's heads (runs of 8700):
+// 4.7e-7 without, 4.0e-7 at 16 passes, 3.6e-7 at 4 (uniform chunks of 768
+// rows: 3.8e-7); over seven batches of the three shapes the mean is 0.99 of
+// the uniform chunks'.  At 2 and 1 passes it is 0.98 and TinyLlama's batches
+// are 6-9% slower.
+constexpr int kFlatFlushPasses = 4;
+
+// Segment (workgroup w, item i) has record w + i among its XCD's: along the
+// rows w and i only grow, and one of them grows from a segment to the next,
+// so an item's segments have consecutive records.  After the n_wg + n_items
+// of them come the records of first-level sub-groups (flat_sub_record: the
+// item's first, from its first segment's record).
+__host__ __device__ constexpr int flat_sub_record(int n_wg, int n_items, int rec0, int item)
+{
+    return n_wg + n_items + rec0 / kSubGroup + item;
+}
+__host__ __device__ constexpr int flat_records(int n_wg, int n_items)
+{
+    return flat_sub_record(n_wg, n_items, n_wg + n_items, n_items) + 1;
+}
+
+// Rows [begin, end) of item `item`, whose sequence is at position pos, as
+// chunk lc of n_local of them; rec0: the item's first chunk's record.
+struct FlatSegment {
+    int item, pos, lc, n_local, begin, end, rec0;
+};
+// The segment of workgroup w's run [at, stop) in the item that counts rows
+// [item_begin, item_end), start_rows of them ahead of its first row; an empty
+// one (begin == end) if the run ends before that row.
+__host__ __device__ __forceinline__ FlatSegment flat_segment(int w, int run, int at, int stop, int item,
+                                                             int item_begin, int item_end, int start_rows)
+{
+    const int row0 = item_begin + start_rows;  // the item's first row
+    const int b = at > row0 ? at : row0, e = stop < item_end ? stop : item_end;
+    if (e <= b) return FlatSegment{item, 0, 0, 0, 0, 0, 0};
+    const int w_first = (int)((unsigned)row0 / (unsigned)run), w_last = (int)((unsigned)(item_end - 1) / (unsigned)run);
+    return FlatSegment{item, item_end - row0 - 1, w - w_first, w_last - w_first + 1, b - row0, e - row0, w_first + item};
+}
+
 // Rows of one wave sub-tile: 16 (two MFMA row sets), i.e. 16 KiB of K and V
 // at head_dim 128, whatever the number of q heads per KV head.
 __host__ __device__ constexpr int subtile_rows(int hd, int g) { return (void)hd, (void)g, 16; }
@@ -589,9 +649,11 @@ struct NewRow {
     bool on;
 };
 
-template <int HD, int G, int NW, bool MFMA, bool PART, int KVS>
+// FLAT: the body serves one segment of a flat launch, fs; a workgroup runs it
+// once per segment.
+template <int HD, int G, int NW, bool MFMA, bool PART, int KVS, bool FLAT = false>
 __device__ __forceinline__ void decode_attention_body(const StepArgs &args, const Preload &pre, Timeline &tl,
-                                                      NewRow &nr)
+                                                      NewRow &nr, const FlatSegment &fs = FlatSegment{})
 {
     using S = Shape<HD, G, NW>;
     constexpr int GQ = S::GQ, NF = S::NF, R = S::R, KS = S::KS;
@@ -622,11 +684,11 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     const int spread_log2 = (int)((pre.w0 >> 14) & 3u);
     const int n_kv_heads = (int)(pre.w0 >> 16);
     const int lq = (int)fast_div((uint32_t)local, FastDiv{pre.m_gc, (pre.w0 >> 10) & 15u});
-    const int lc = local - lq * grid_chunks;
-    const int pgroup = lq * kXcds + xcd;
-    const int group = pgroup >> spread_log2;
-    const int part = pgroup & ((1 << spread_log2) - 1);
-    const int chunk_id = part * grid_chunks + lc;  // within the group
+    const int lc = FLAT ? fs.lc : local - lq * grid_chunks;
+    const int pgroup = (FLAT ? fs.item : lq) * kXcds + xcd;
+    const int group = FLAT ? pgroup : pgroup >> spread_log2;
+    const int part = FLAT ? 0 : pgroup & ((1 << spread_log2) - 1);
+    const int chunk_id = FLAT ? lc : part * grid_chunks + lc;  // within the group
     // The sequence, its position, its chunks (chunk c starts at
     // min(c cq + min(c, cr), T)) and its slab: from the preloaded words for
     // one sequence at a host position, else from the argument block, whose
@@ -636,7 +698,13 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     // after another.
     int seq, pos, n_chunks, cq, cr;
     size_t slab;
-    if (pre.w1 != kPreGeneral) {
+    if constexpr (FLAT) {
+        seq = (int)fast_div((uint32_t)group, args.by_kv_heads);
+        pos = fs.pos;
+        n_chunks = fs.n_local;
+        cq = cr = 0;
+        slab = (size_t)seq * (size_t)args.seq_stride;
+    } else if (pre.w1 != kPreGeneral) {
         if (group >= n_kv_heads) return;
         seq = 0;
         pos = (int)(pre.w1 & (kPreLimit - 1));
@@ -682,14 +750,17 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     const KvGroup kg = KVS ? kv_group<G>(kvv, n_kv_heads, KVS) : KvGroup{kvv, 0, kvv * G};
     const int kvh = kg.kvh;
     const bool store_new = kg.half == 0;  // the one group per cache head that appends the new token
-    const int tid = threadIdx.x;
+    int tid = threadIdx.x;
+    // (what follows from the thread's number is worked out again for each
+    // segment: held through the ones before, it took 256 registers and scratch)
+    if constexpr (FLAT) asm volatile("" : "+v"(tid));
     const int wave = tid / kWave;
     const int lane = tid % kWave;
 
     const int T = pos + 1;
     if (chunk_id >= n_chunks) return;
     // chunks of this part (at least 1 here)
-    const int n_local = min(grid_chunks, n_chunks - part * grid_chunks);
+    const int n_local = FLAT ? n_chunks : min(grid_chunks, n_chunks - part * grid_chunks);
 
     const int kv_dim = (n_kv_heads >> KVS) * HD;
     const int q_dim = n_kv_heads * G * HD;  // every q head of a sequence
@@ -704,8 +775,8 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     constexpr int LAST_NEW = NEW_AFTER ? 1 : 0;
     int chunk_begin, chunk_end, row_end, last;
     if constexpr (PART) {
-        chunk_begin = min(chunk_id * cq + min(chunk_id, cr), T);
-        chunk_end = min((chunk_id + 1) * cq + min(chunk_id + 1, cr), T);
+        chunk_begin = FLAT ? fs.begin : min(chunk_id * cq + min(chunk_id, cr), T);
+        chunk_end = FLAT ? fs.end : min((chunk_id + 1) * cq + min(chunk_id + 1, cr), T);
         row_end = min(pos, chunk_end);
         last = min(pos - LAST_NEW, chunk_end - 1);
     } else {
@@ -725,6 +796,9 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     __shared__ float4 comb_o[NW][RPV][G][D4];
     __shared__ __align__(16) float comb_l[G][NW];  // [head][wave]: a head's NW values in one read
     __shared__ __align__(16) float comb_m[G][NW];
+    // FLAT: the new token's staging, apart from the combine buffer, which holds
+    // the waves' flushed sums during the loop
+    __shared__ float4 stage_lds[FLAT ? NW : 1][FLAT ? 2 * D4 : 1];
     __shared__ float2 ml_lds[GM * kFinalMax];  // the asymmetric merge's final (max, sum) pairs
     __shared__ int s_last;
 
@@ -841,7 +915,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     // The table row, for the new token's k, in this wave's combine buffer
     // (unused until the waves combine): float4 [D4, 2*D4); the k_new row
     // goes to [0, D4) when it is needed.
-    float4 *nt_lds = &comb_o[wave][0][0][0];
+    float4 *nt_lds = FLAT ? &stage_lds[FLAT ? wave : 0][0] : &comb_o[wave][0][0][0];
     static_assert(RPV * G >= 2, "new-token staging");
     if (lane < HD / 2) reinterpret_cast<float2 *>(nt_lds + D4)[lane] = qt[0];
     __syncthreads();
@@ -870,7 +944,35 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
 #pragma unroll
         for (int e = 0; e < 4; e++) acc[q][e] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+    // FLAT: this wave's outputs so far, relative to 2^m_sum, as its partials in
+    // the combine buffer (m_sum: -inf before the first)
+    float m_sum[FLAT ? G : 1];
+    if constexpr (FLAT) {
+#pragma unroll
+        for (int h = 0; h < G; h++) m_sum[h] = -INFINITY;
+    }
+    bool flushed = false;
+    auto flush = [&]() {
+#pragma unroll
+        for (int h = 0; h < G; h++) {
+            float4 o = make_float4(acc[h / 4][0][h % 4], acc[h / 4][1][h % 4], acc[h / 4][2][h % 4], acc[h / 4][3][h % 4]);
+            if (flushed) fma4(o, m_sum[h] == -INFINITY ? 0.0f : fast_exp2(m_sum[h] - m_ref[h]), comb_o[wave][vg][h][vj]);
+            comb_o[wave][vg][h][vj] = o;
+            m_sum[h] = m_ref[h];
+        }
+        flushed = true;
+    };
+
     for (int i = 0; i < n_sub; i++) {
+        if constexpr (FLAT) {
+            if (i > 0 && i % kFlatFlushPasses == 0) {
+                flush();
+#pragma unroll
+                for (int q = 0; q < GQ; q++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[q][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
         const int sub = sub0 + i < n_sub ? sub0 + i : sub0 + i - n_sub;
         const int base = chunk_begin + (sub * NW + wave) * R;
         // A later pass whose rows for this wave all lie past the chunk's end
@@ -1134,6 +1236,9 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     }
 
     // Per-wave partials to LDS: every V row slot its own accumulator.
+    if constexpr (FLAT) {
+        flush();
+    } else
 #pragma unroll
     for (int h = 0; h < G; h++)
         comb_o[wave][vg][h][vj] = make_float4(acc[h / 4][0][h % 4], acc[h / 4][1][h % 4],
@@ -1151,11 +1256,15 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
 
     // Combine the waves: one float4 of one head per thread.
     const bool single = (n_local == 1);
-    const int n_rec = records_per_head(grid_chunks);
-    const size_t ws_head0 = (size_t)pgroup * G * (size_t)n_rec;
+    // (a flat launch's records: those of an XCD's segments together)
+    const int n_items = FLAT ? (a.n_groups + kXcds - 1) / kXcds : 0;
+    const int n_rec = FLAT ? flat_records(grid_chunks, n_items) : records_per_head(grid_chunks);
+    const size_t ws_head0 = (size_t)(FLAT ? xcd : pgroup) * G * (size_t)n_rec;
+    const int rec0 = FLAT ? fs.rec0 : 0;                    // the group's first chunk's record
+    const int sub_rec0 = FLAT ? flat_sub_record(grid_chunks, n_items, rec0, fs.item) : grid_chunks;  // its first sub-group's
     // A part-group's finished result: the output row (one part), or the
     // part's unnormalised record for the cross-XCD merge launch.
-    const bool parts = spread_log2 > 0;
+    const bool parts = !FLAT && spread_log2 > 0;
     auto emit = [&](int head, int col, float4 o, float M, float L) {
         if (parts) {
             reinterpret_cast<float4 *>(a.ws_po + ((size_t)pgroup * G + head) * HD)[col] = o;
@@ -1200,7 +1309,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
             emit(ch, cd4, o, M, L);
         } else {
             // Partial o and (max, sum), into this XCD's L2.
-            const uint32_t row = (uint32_t)(ch * n_rec + lc);
+            const uint32_t row = (uint32_t)(ch * n_rec + rec0 + lc);
             buf_store4(wo_rsrc, row * (HD * 4u) + 16u * cd4, o);
             if (cd4 == 0) buf_store2(wm_rsrc, row * 8u, make_float2(M, L));
         }
@@ -1514,7 +1623,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
         __syncthreads();
         tl.mark(kTlCounted);
         const int prev = s_last;
-        final_fold(0, std::integral_constant<int, NC>{}, n_local, prev);
+        final_fold(rec0, std::integral_constant<int, NC>{}, n_local, prev);
     };
     if (!(a.merge_asym & 1) && n_local > 1) {
         if (n_local <= 8) return merge_flat(std::integral_constant<int, 8>{});
@@ -1531,7 +1640,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
             if (n_local <= 40) return merge_flat(std::integral_constant<int, 40>{});
         }
     }
-    if (a.merge_asym & 1) {
+    if (!FLAT && (a.merge_asym & 1)) {
         if constexpr (32 + 4 <= MG * BW) {
             if (n_local == 64) return merge_asym(std::integral_constant<int, 64>{});
         }
@@ -1562,7 +1671,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     if (tid == 0) ctr[(1 + sg) * kCtrStride] = 0;
     float4 ox;
     float Mx, Lx;
-    fold(sg * kSubGroup, sg_n, ox, Mx, Lx);
+    fold(rec0 + sg * kSubGroup, sg_n, ox, Mx, Lx);
     if (n_sg == 1) {
         if (mg == 0 && live) emit(mh, md4, ox, Mx, Lx);
         tl.role(kTlRoleFinal, 0);
@@ -1570,7 +1679,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
         return;
     }
     if (mg == 0 && live) {
-        const uint32_t row = (uint32_t)(mh * n_rec + grid_chunks + sg);
+        const uint32_t row = (uint32_t)(mh * n_rec + sub_rec0 + sg);
         buf_store4(wo_rsrc, row * (HD * 4u) + 16u * md4, ox);
         if (md4 == 0) buf_store2(wm_rsrc, row * 8u, make_float2(Mx, Lx));
     }
@@ -1588,7 +1697,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     if (!s_last) return;
     tl.role(kTlRoleFinal, n_sg - 1);
     if (tid == 0) ctr[0] = 0;
-    fold(grid_chunks, n_sg, ox, Mx, Lx);
+    fold(sub_rec0, n_sg, ox, Mx, Lx);
     if (mg == 0 && live) emit(mh, md4, ox, Mx, Lx);
     tl.mark(kTlFolded);
 }
@@ -1604,6 +1713,103 @@ __global__ __launch_bounds__(NW * kWave, (MFMA && G == 8 && HD == 128) ? 2 : 1) 
     if (nr.on) {
         *reinterpret_cast<float4 *>(nr.kdst) = nr.k;
         *reinterpret_cast<float4 *>(nr.vdst) = nr.v;
+    }
+#ifdef LEAP_TIMELINE
+    tl.mark(kTlEnd);
+    tl.flush(a.tl);
+#endif
+}
+
+// Inclusive prefix sum over the 64 lanes of a wave (DPP: within the 16-lane
+// rows, then row 0 into row 1 and row 2 into row 3, then the lower half into
+// the upper).
+__device__ __forceinline__ int wave_prefix_sum(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);  // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);  // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);  // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31
+    return v;
+}
+
+// The decode kernel for a batch whose groups do not cut evenly over the CUs
+// (see kFlatSegmentRows; the host's rule: flat_launch).  StepArgs::grid_chunks
+// is the workgroups per XCD, StepArgs::chunk the rows that an item's start
+// counts as; at most kFlatMaxItems items per XCD.
+// What bounds it is the CU with the most to take in, then the merge.  Graph
+// replay, us per launch, uniform chunks (at the host's choice) -> flat:
+// Llama-3-8B heads, 16 sequences of 200-2000 rows 33.3 -> 29.2 (145 MB, 4.35
+// -> 4.96 TB/s), 8 of them 23.2 -> 18.0, 6 of 400-4000 rows 29.2 -> 24.1, 64
+// of 400-4000 189.5 -> 175.2; 12 sequences of 2000 rows 46.9 -> 37.3 and of
+// 8000 164.7 -> 122.5; Llama-3-70B heads, 16 of 200-2000 rows 45.3 -> 32.2;
+// TinyLlama heads, 64 of 200-2000 rows 50.7 -> 33.2.
+template <int HD, int G, int NW, int KVS>
+__global__ __launch_bounds__(NW * kWave, (G == 8 && HD == 128) ? 2 : 1) void decode_attention_flat_kernel(LEAP_PRELOAD_PARAMS, StepArgs a)
+{
+    Timeline tl;
+    tl.mark(kTlStart);
+    const int xcd = blockIdx.x % kXcds, w = blockIdx.x / kXcds;
+    __shared__ int2 items_lds[NW][kWave];  // per wave: each item's rows and the rows up to its end
+    asm volatile("" ::"s"(a.pos_dev), "s"(a.max_pos), "s"(a.seq_len), "s"(a.n_groups), "s"(a.grid_chunks),
+                 "s"(a.chunk), "s"(a.by_kv_heads.m), "s"(a.by_kv_heads.s), "s"(a.by_grid_chunks.m),
+                 "s"(a.by_grid_chunks.s));
+    const int n_wg = a.grid_chunks, start_rows = a.chunk;
+    const int n_items = (a.n_groups - xcd + kXcds - 1) / kXcds;
+    int at, stop, run;
+    {
+        // Every wave works out the XCD's rows and the workgroup's run by
+        // itself: lane i has item i's rows, 0 for a position the launch
+        // cannot serve.
+        const int i = threadIdx.x % kWave;
+        int rows = 0;
+        if (i < n_items) {
+            const int pos = a.pos_dev[fast_div((uint32_t)(i * kXcds + xcd), a.by_kv_heads)];
+            if (pos >= 0 && pos < a.seq_len && pos <= a.max_pos) rows = pos + 1 + start_rows;
+        }
+        const int upto = wave_prefix_sum(rows);
+        const int total = __builtin_amdgcn_readlane(upto, kWave - 1);
+        run = max((int)fast_div((uint32_t)(total + n_wg - 1), a.by_grid_chunks), kFlatMinRun);
+        at = w * run;
+        stop = min(at + run, total);
+        items_lds[threadIdx.x / kWave][i] = make_int2(rows, upto);
+        // The output rows of a sequence whose position the launch cannot
+        // serve read NaN (item i by workgroup i mod n_wg).
+        for (uint64_t bad = __builtin_amdgcn_ballot_w64(i < n_items && rows == 0); bad; bad &= bad - 1) {
+            const int item = __builtin_ctzll(bad);
+            if (item % n_wg != w) continue;
+            const int group = item * kXcds + xcd, seq = (int)fast_div((uint32_t)group, a.by_kv_heads);
+            const int kvv = group - seq * a.n_kv_heads;
+            const int qh0 = KVS ? kv_group<G>(kvv, a.n_kv_heads, KVS).qh0 : kvv * G;
+            for (int j = threadIdx.x; j < G * HD; j += NW * kWave)
+                a.out[(size_t)seq * a.n_heads * HD + (size_t)qh0 * HD + j] = __builtin_nanf("");
+        }
+    }
+    while (at < stop) {
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int2 it = items_lds[tid / kWave][tid % kWave];
+        // the item that row `at` counts in: the first to end past it
+        const int item = __builtin_ctzll(__builtin_amdgcn_ballot_w64(it.y > at));
+        const int item_end = __builtin_amdgcn_readlane(it.y, item);
+        const FlatSegment fs = flat_segment(w, run, at, stop, item, item_end - __builtin_amdgcn_readlane(it.x, item),
+                                            item_end, start_rows);
+        at = item_end;
+        if (fs.begin == fs.end) continue;
+        NewRow nr;
+        nr.on = false;
+        // (the arguments are read again for each segment, rather than held in
+        // scalar registers through the ones before)
+        const StepArgs la = late_args(a, kArgsOffset);
+        const Preload pre{la.q, la.k_new, la.k_cache, la.v_cache, la.rope, 0u,
+                          (uint32_t)la.grid_chunks | ((uint32_t)la.n_kv_heads << 16), 0u, 0u};
+        decode_attention_body<HD, G, NW, true, true, KVS, true>(la, pre, tl, nr, fs);
+        if (nr.on) {
+            *reinterpret_cast<float4 *>(nr.kdst) = nr.k;
+            *reinterpret_cast<float4 *>(nr.vdst) = nr.v;
+        }
+        __syncthreads();  // the workgroup's LDS is free
     }
 #ifdef LEAP_TIMELINE
     tl.mark(kTlEnd);

@@ -3,6 +3,7 @@
 //   - kernels_decode.hip: the measurement kernels with the decode kernel's
 //     grids and the cross-XCD merge; kernels_decode_{64,64p,128,128p}.hip:
 //     the decode-attention kernels by head_dim and instance kind;
+//     kernels_decode_{64,128}f.hip: the flat kernels (batches) by head_dim;
 //   - kernels_gemv.hip: the fp32 projection GEMVs by model width;
 //   - kernels_q8.hip: the int8 W8A8 projection GEMVs by width, group size,
 //     rows per team and input kind.
@@ -62,6 +63,13 @@ extern template KernelFn pick_decode<64, false>(int, bool, int, int);
 extern template KernelFn pick_decode<64, true>(int, bool, int, int);
 extern template KernelFn pick_decode<128, false>(int, bool, int, int);
 extern template KernelFn pick_decode<128, true>(int, bool, int, int);
+
+// The flat decode kernel for g q heads per launch group (kvs: 1 for 16 q
+// heads per KV head as two groups of 8); nullptr for a shape without one.
+template <int HD>
+KernelFn pick_flat(int g, int kvs);
+extern template KernelFn pick_flat<64>(int, int);
+extern template KernelFn pick_flat<128>(int, int);
 
 // The cross-XCD merge of a spread launch.
 MergeFn pick_merge(int hd, int g);

@@ -75,6 +75,7 @@ struct leap_hip_attention {
     int split = 0;
     int n_cu = 256;  // compute units of the device
     int max_chunks = 1;  // chunks per sequence the workspace holds records for
+    int max_flat = 0;    // workgroups per XCD of a flat launch it holds records for
     bool valu = false;   // score and weighted-V products on the VALU (measurement knob)
     int fold_helper = 1; // 1: two workgroups share a one-level merge's final fold; 0: the last alone; 2: test of the fallback
     std::string err;
@@ -170,7 +171,9 @@ struct LaunchShape {
     bool ws_parts = true;  // the buffers hold part records and kXcds part-groups' records
     int fold_helper = 1;   // leap_hip_attention_set_fold_helper
     int kv_split = 0;      // 2^kv_split launch groups per cache head (kv_view's, launch_view's)
+    int max_flat = 0;      // workgroups per XCD of a flat launch that the buffers hold records and counters for
 };
+
 
 // The device buffers of one launch (one layer): the cache slabs of sequence
 // 0 at this layer and the distance between sequences, the RoPE table, and
@@ -194,6 +197,7 @@ LaunchShape shape_of(const leap_hip_attention *h)
                   h->n_cu, h->split, h->max_chunks, h->valu};
     s.fold_helper = h->fold_helper;
     s.kv_split = v.kv_split;
+    s.max_flat = h->max_flat;
     return s;
 }
 
@@ -422,6 +426,102 @@ long long g_tl_launches = 0;
 constexpr size_t kTlRingWords = (size_t)leap::kTlSlots * leap::kTlMaxWgs * leap::kTlPoints;
 #endif
 
+// Workgroups per XCD of a flat launch (decode_attention_flat_kernel) for a
+// batch, or 0 where the uniform chunks above serve it.
+//   - Equal lengths: the uniform chunks leave CUs without their share when
+//     the groups do not divide them (Llama-3-8B: 12 sequences run 36 chunks
+//     on an XCD's 32 CUs).  Flat once less than 3/4 of the CUs' time is used,
+//     or 9/10 with 8 q heads per KV head, whose products overlap better with
+//     two workgroups per CU.  Graph replay, us per launch, uniform -> flat:
+//     Llama-3-8B heads, 12 sequences of 2000 rows 46.9 -> 37.3, 3 of 4000
+//     27.6 -> 21.9 (33 chunks on 32 CUs); 6 (15/16 used) of 4000 35.2 ->
+//     37.5; 24 (3/4) of 1000-8000 36.7 -> 40.5 to 234.6 -> 232.7; 70B heads,
+//     12 of 2000 49.9 -> 40.1, 24 of 8000 276 -> 253.
+//     TinyLlama's heads (8 per KV head at head_dim 64), where the uniform
+//     chunks run one workgroup per CU, are bound by their products and take
+//     two: 32 sequences of 1000 rows 22.1 -> 18.7, of 4000 65.4 -> 49.5, 16 of
+//     1000 14.1 -> 12.8 (with the runs cut at the sequences' ends), but 8 of
+//     1000 (62 rows a run) 10.1 -> 14.1.
+//   - Ragged lengths: flat once a run holds kFlatRun rows (a shorter one
+//     costs more in starts and records than the even cut saves: Llama-3-8B
+//     heads, 24 of 30-300 rows (62 a run) 12.1 -> 13.2, 16 of 100-1000 (137)
+//     23.2 -> 18.1; 70B heads, 8 of 100-1000 (69) 13.9 -> 14.8, 12 (103) 21.1
+//     -> 17.5).  With one q head per KV head the uniform chunks measured as
+//     fast (the mean of 29 batches -0.3%).
+// Two workgroups per CU, but one for 4 q heads per KV head or fewer from
+// kFlatOneBytes on: Llama-3-8B heads, 64 sequences of 400-4000 rows (1.2 GB)
+// 181.3 -> 175.2, 32 of 800-8000 177.9 -> 174.0; 12 of 400-4000 (210 MB)
+// 39.2 -> 41.2.
+constexpr int kFlatPerCu = 2;
+constexpr long long kFlatOneBytes = 512ll << 20;
+bool equal_lengths(int n_seq, long long total_rows, int max_T) { return total_rows == (long long)n_seq * max_T; }
+int flat_launch(const LaunchShape &s, int n_seq, long long total_rows, int max_T)
+{
+    const long long n_groups = (long long)n_seq * s.n_kv_heads;
+    if (s.valu || s.split > 0 || s.max_flat < kFlatPerCu * s.n_cu / leap::kXcds) return 0;
+    if (n_groups < 2 * leap::kXcds || n_groups > leap::kFlatMaxItems * leap::kXcds) return 0;
+    const int cus = s.n_cu / leap::kXcds;
+    const int items = (int)((n_groups + leap::kXcds - 1) / leap::kXcds);
+    const long long bytes = total_rows * (long long)s.n_kv_heads * s.head_dim * 8ll;
+    const int per_cu = s.group <= 4 && bytes >= kFlatOneBytes ? 1 : kFlatPerCu;
+    if (equal_lengths(n_seq, total_rows, max_T)) {
+        if (s.group == 8 && s.head_dim == 64 && kFlatPerCu * cus % items == 0)
+            return (long long)max_T * items >= 120ll * kFlatPerCu * cus ? kFlatPerCu * cus : 0;
+        const int even = even_chunks_for(s, n_seq, total_rows, max_T);
+        const int chunk = choose_chunk(s, n_seq, total_rows, max_T);
+        const long long wgs = (long long)items * (even ? even : (max_T + chunk - 1) / chunk);
+        if (wgs < 3 * cus / 4) return 0;  // small: the launch leaves CUs out on purpose
+        const long long rounds = (wgs + cus - 1) / cus;
+        return wgs * (s.group == 8 ? 10 : 4) < rounds * cus * (s.group == 8 ? 9 : 3) ? per_cu * cus : 0;
+    }
+    const int min_run = s.group == 8 ? 96 : 64;
+    return s.group > 1 && total_rows * s.n_kv_heads >= (long long)min_run * kFlatPerCu * s.n_cu ? per_cu * cus : 0;
+}
+
+// Enqueue a flat launch of n_wg workgroups per XCD.
+hipError_t launch_flat(const LaunchShape &s, const LaunchBuffers &b, int n_wg, int n_seq, const int *pos_dev,
+                       int max_pos, long long total_rows, const float *q, const float *k, const float *v, float *out,
+                       hipStream_t stream)
+{
+    KernelFn fn = s.head_dim == 64 ? pick_flat<64>(s.group, s.kv_split) : pick_flat<128>(s.group, s.kv_split);
+    if (!fn || s.n_kv_heads >= 65536) return hipErrorInvalidValue;
+    leap::StepArgs a{};
+    a.q = q;
+    a.k_new = k;
+    a.v_new = v;
+    a.out = out;
+    a.k_cache = b.k_cache;
+    a.v_cache = b.v_cache;
+    a.rope = b.rope;
+    a.pos_dev = pos_dev;
+    a.ws_o = b.ws_o;
+    a.ws_ml = b.ws_ml;
+    a.counters = b.counters;
+    a.seq_stride = b.seq_stride;
+    a.max_pos = max_pos;
+    a.seq_len = s.seq_len;
+    a.n_heads = s.n_heads;
+    a.n_kv_heads = s.n_kv_heads;
+    a.grid_chunks = n_wg;
+    a.n_groups = n_seq * s.n_kv_heads;
+    // Equal lengths that the runs divide are cut at the sequences' ends when
+    // a start counts as no rows.
+    const int items = (a.n_groups + leap::kXcds - 1) / leap::kXcds;
+    a.chunk = equal_lengths(n_seq, total_rows, max_pos + 1) && n_wg % items == 0 ? 0 : leap::kFlatSegmentRows;
+    a.scale_log2 = (float)(1.4426950408889634 / std::sqrt((double)s.head_dim));
+    a.by_grid_chunks = leap::make_fastdiv((uint32_t)n_wg);
+    a.by_kv_heads = leap::make_fastdiv((uint32_t)s.n_kv_heads);
+    a.by_chunk = a.by_even = leap::make_fastdiv(1u);
+    a.kv_split = s.kv_split;
+#ifdef LEAP_TIMELINE
+    a.tl = g_tl_ring ? g_tl_ring + (size_t)(g_tl_launches++ % leap::kTlSlots) * leap::kTlMaxWgs * leap::kTlPoints
+                     : nullptr;
+#endif
+    const leap::Preload p = leap::make_preload(a, false);
+    return launch_k(fn, dim3((unsigned)(n_wg * leap::kXcds)), dim3((unsigned)kThreads), stream, p.q, p.k_new, p.k_cache,
+                    p.v_cache, p.rope, p.m_gc, p.w0, p.w1, p.w2, a);
+}
+
 // Enqueue one decode-attention launch.  Returns 0, or a HIP error code
 // (hipErrorInvalidValue for a shape without a kernel or a launch too large).
 hipError_t launch_attention(const LaunchShape &shape, const LaunchBuffers &b, int n_seq, const int *pos_dev,
@@ -430,6 +530,9 @@ hipError_t launch_attention(const LaunchShape &shape, const LaunchBuffers &b, in
 {
     const LaunchShape s = launch_view(shape, n_seq, total_rows);
     const int hd = s.head_dim;
+    if (kind == kDecode && pos_dev)
+        if (const int n_wg = flat_launch(s, n_seq, total_rows, max_pos + 1))
+            return launch_flat(s, b, n_wg, n_seq, pos_dev, max_pos, total_rows, q, k, v, out, stream);
     const int even = even_chunks_for(s, n_seq, total_rows, max_pos + 1);
     const int chunk = even ? (max_pos + even) / even : choose_chunk(s, n_seq, total_rows, max_pos + 1);
     // Chunks of at most half a pass (the short contexts' half-pass chunks,
@@ -703,6 +806,8 @@ hipError_t load_kernel_tables()
         reinterpret_cast<const void *>(pick_kernel(64, 4, kDecode, false, true, false)),
         reinterpret_cast<const void *>(pick_kernel(128, 4, kDecode, false, false, false)),
         reinterpret_cast<const void *>(pick_kernel(128, 4, kDecode, false, true, false)),
+        reinterpret_cast<const void *>(pick_flat<64>(4, 0)),
+        reinterpret_cast<const void *>(pick_flat<128>(4, 0)),
         reinterpret_cast<const void *>(pick_kernel(128, 4, kFloorLaunch, false, false, false)),
         reinterpret_cast<const void *>(pick_q8(4096, 64, leap::kQ8InRms, 6144, 256, &rpt)),
     };
@@ -854,7 +959,12 @@ int leap_hip_attention_create(const leap_hip_attention_config *cfg, leap_hip_att
     const KvView kvv = kv_view(h->group, c.n_kv_heads);
     h->max_chunks = max_chunks_for(c.seq_len, c.head_dim, kvv.group, kvv.n_kv_heads, h->n_cu, leap::kMaxChunks);
     const size_t n_pg = std::max<size_t>((size_t)c.max_batch * kvv.n_kv_heads, leap::kXcds);
-    const size_t ws_rows = n_pg * kvv.group * leap::records_per_head(h->max_chunks);
+    // (and a flat launch's: records per XCD for its workgroups and at most
+    // kFlatMaxItems groups)
+    const int items = (int)std::min<size_t>((n_pg + leap::kXcds - 1) / leap::kXcds, leap::kFlatMaxItems);
+    if (items >= 2) h->max_flat = kFlatPerCu * h->n_cu / leap::kXcds;
+    const size_t ws_rows = std::max(n_pg * kvv.group * leap::records_per_head(h->max_chunks),
+                                    (size_t)leap::kXcds * kvv.group * leap::flat_records(h->max_flat, items));
     CREATE_TRY(hipMalloc(&h->ws_o, ws_rows * c.head_dim * sizeof(float)));
     CREATE_TRY(hipMalloc(&h->ws_ml, ws_rows * sizeof(float2)));
     // (launch_view's two groups of 2 or 4 q heads per cache head, or four of
@@ -862,7 +972,7 @@ int leap_hip_attention_create(const leap_hip_attention_config *cfg, leap_hip_att
     // 4 or 8)
     const bool twins = (kvv.group == 8 || kvv.group == 4) && kvv.kv_split == 0;
     const size_t n_ctr = std::max<size_t>(n_pg, twins ? 2 * leap::kXcds : 0);
-    h->counter_bytes = n_ctr * leap::counters_per_group(h->max_chunks) * sizeof(int);
+    h->counter_bytes = n_ctr * leap::counters_per_group(std::max(h->max_chunks, h->max_flat)) * sizeof(int);
     CREATE_TRY(hipMalloc(&h->ws_po, (size_t)leap::kXcds * h->group * c.head_dim * sizeof(float)));
     CREATE_TRY(hipMalloc(&h->ws_pml, (size_t)leap::kXcds * h->group * sizeof(float2)));
     CREATE_TRY(hipMalloc(&h->counters, h->counter_bytes));
