@@ -10,12 +10,13 @@
 //     quantized per group, then x += Wo . that (the wo matmul and the residual
 //     after the attention block).
 //
-// One workgroup per CU: the fp32 input vector (and the rms weight) is read,
-// normalised and quantized once per workgroup and shared through LDS, so that
-// the int8 weights, which are a quarter of the fp32 bytes per row, are not
-// outweighed by every workgroup re-reading 16-32 KiB of activations from L2.
-// A row's int8 load is one contiguous E-byte access per thread (E = n/256; 1
-// KiB per wave at n = 4096).
+// One workgroup per CU where the rows allow it: the fp32 input vector (and the
+// rms weight) is read, normalised and quantized once per workgroup and shared
+// through LDS, so that the int8 weights, which are a quarter of the fp32 bytes
+// per row, are not outweighed by every workgroup re-reading 16-32 KiB of
+// activations from L2.  A wave takes whole rows (or halves of them at n =
+// 8192): each load instruction reads 1 KiB of one row contiguously, and every
+// width that is a multiple of 1024 uses every lane.
 //
 // Arithmetic, matched to the reference bit for bit:
 //   - group scale sx = max|v| * (1/127) (the reference's release build folds
@@ -99,284 +100,208 @@ __device__ __forceinline__ float group_max_w(float v)
     }
 }
 
-// E int8 values per thread as E/4 packed words.
-template <int E>
-struct Q8Row {
-    int v[E / 4];
-};
-
-// The same E bytes through a raw buffer load (non-temporal): `off` past the
-// descriptor's range reads zeros without touching memory, which keeps the
-// load unconditional for lanes that own no values.
-template <int E>
-__device__ __forceinline__ Q8Row<E> load_row_buf(__amdgpu_buffer_rsrc_t r, uint32_t off)
-{
-    Q8Row<E> w;
-    if constexpr (E == 8) {
-        const u32x2 a = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, kNt);
-        w.v[0] = (int)a.x;
-        w.v[1] = (int)a.y;
-    } else {
-#pragma unroll
-        for (int c = 0; c < E / 16; c++) {
-            const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off + 16u * c), 0, kNt);
-            w.v[4 * c] = (int)a.x;
-            w.v[4 * c + 1] = (int)a.y;
-            w.v[4 * c + 2] = (int)a.z;
-            w.v[4 * c + 3] = (int)a.w;
-        }
-    }
-    return w;
-}
-
-template <int E>
-__device__ __forceinline__ Q8Row<E> load_row_nt(const int8_t *p)
-{
-    Q8Row<E> r;
-    if constexpr (E == 8) {
-        typedef int i2 __attribute__((ext_vector_type(2)));
-        const i2 a = __builtin_nontemporal_load(reinterpret_cast<const i2 *>(p));
-        r.v[0] = a.x;
-        r.v[1] = a.y;
-    } else {
-        typedef int i4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-        for (int c = 0; c < E / 16; c++) {
-            const i4 a = __builtin_nontemporal_load(reinterpret_cast<const i4 *>(p) + c);
-            r.v[4 * c] = a.x;
-            r.v[4 * c + 1] = a.y;
-            r.v[4 * c + 2] = a.z;
-            r.v[4 * c + 3] = a.w;
-        }
-    }
-    return r;
-}
-
-constexpr int kQ8Threads = 1024;  // one workgroup per CU: 16 waves
-constexpr int kQ8Teams = kQ8Threads / kGemvThreads;
-constexpr int kQ8Waves = kQ8Threads / 64;
-
-// One workgroup of 1024 threads (16 waves, one per CU at the launch sizes
-// used) owns rows [row0, row0 + 4*RPT): four teams of 256 threads, team k
-// taking rows row0 + k*RPT + j, j < RPT.  In a team, thread t < ACT owns the
-// E = n/ACT values [t*E, t*E + E) of each of its rows, so a group of gs values
-// is L = gs/E adjacent lanes.  ACT is 256 when n is 256 times a power of two;
-// for n = 3072 (ACT 192, E 16) and 5120 (ACT 160, E 32) the team's last
-// threads own no values: their row loads read zeros past the range and they
-// write nothing.  The input vector is read, normalised and quantized once per
-// workgroup, each of the first 4*ACT threads taking E/4 consecutive values,
-// and shared through LDS.
+// A workgroup of NWV waves owns rows [row0, row0 + per_wg), per_wg <= J * NWV /
+// WPR: teams of WPR waves, team t taking rows row0 + t + j * NWV / WPR, j < J.
+// Wave p of a team holds the row's 1 KiB pieces [p * NL / WPR, (p + 1) * NL /
+// WPR) of n = NL * 1024 values, 16 a lane, so a group of gs values is L = gs/16
+// adjacent lanes.  The host picks (J, NWV, WPR) from the rows per CU
+// (pick_q8), so that each CU has the same number of rows and the waves of a
+// workgroup nearly so; rows past the workgroup's read zeros (an offset past
+// the descriptor's range) and write slots that nobody reads.
 //
-// Issue order: the input first, then the team's scales and weight rows
-// (4*RPT*n bytes per workgroup, 96 KiB for Wq/Wk/Wv at Llama-3-8B), all before
-// anything waits.  RPT is a compile-time count so that every load is
-// unconditional: load waits count outstanding loads in issue order, and with a
-// runtime row count the wait for the input had to assume the longest queue,
-// which made the normalisation wait for every weight row (0.8 us at
-// Llama-3-8B).  The input work now runs while the weights stream.
+// Bounded by the CU's intake: its rows, plus 16-32 KiB of input ahead of
+// them, then the serial tail (dot products, one barrier, the ordered chain of
+// n / gs fused multiply-adds).  Before, teams of four waves took a row and
+// every launch ran 1024 threads; widths that are not 256 times a power of two
+// idled 64-96 of a team's 256 threads, and the rows per team came in steps
+// that left 1.2-1.5 rounds of workgroups at Llama-2's widths.  us per launch,
+// back to back over 1 GiB of weights, before -> now: Llama-3-8B q/k/v (6144 x
+// 4096) 7.29 -> 6.33, wo 5.44 -> 5.05 (the weights alone on the old grid 5.16
+// and 4.05); Llama-2-13B q/k/v (15360 x 5120) 24.4 -> 16.2, wo 9.3 -> 6.8;
+// Llama-2-7B q/k/v (12288 x 4096) 14.3 -> 10.7; Llama-3-70B q/k/v (10240 x
+// 8192) 18.8 -> 17.2, wo 14.2 -> 14.1; TinyLlama q/k/v (2560 x 2048) 4.14 ->
+// 2.95, wo 3.47 -> 2.96; Llama-3.2-3B q/k/v (5120 x 3072) 5.51 -> 5.11, wo
+// 4.40 -> 3.88.
 //
-// Arguments: the input and weight pointers and the row count come first as
+// Issue order: the input first, then the rows' scales and the weight rows
+// (96 KiB a workgroup for Wq/Wk/Wv at Llama-3-8B), all before anything waits.
+// J is a compile-time count so that every load is unconditional: load waits
+// count outstanding loads in issue order, and with a runtime row count the
+// wait for the input had to assume the longest queue, which made the
+// normalisation wait for every weight row (0.8 us at Llama-3-8B).  The input
+// work runs while the weights stream.
+//
+// Arguments: the input and weight pointers and the row counts come first as
 // scalars, which the dispatch preloads into scalar registers (the library is
 // built with -mllvm -amdgpu-kernarg-preload-count=14), so that the first
 // loads do not wait for a load of the arguments; the rest of Q8Args (the
 // outputs) is read after the weight rows are issued (late_args).
-constexpr unsigned kQ8ArgsOffset = 4 * sizeof(void *) + 8;  // Q8Args after the preloaded x, rms_w, w, ws, rows
+constexpr unsigned kQ8ArgsOffset = 4 * sizeof(void *) + 8;  // Q8Args after the preloaded x, rms_w, w, ws, rows, per_wg
 static_assert(alignof(Q8Args) == 8, "argument layout");
-#define LEAP_Q8_PRELOAD_PARAMS const float *pre_x, const float *pre_rms_w, const int8_t *pre_w, const float *pre_ws, int pre_rows
-template <int E, int L, int RPT, int kIn, bool kResid, int ACT = kGemvThreads>
-__global__ __launch_bounds__(kQ8Threads) void q8_gemv_kernel(LEAP_Q8_PRELOAD_PARAMS, Q8Args args)
+#define LEAP_Q8_PRELOAD_PARAMS                                                                                  \
+    const float *pre_x, const float *pre_rms_w, const int8_t *pre_w, const float *pre_ws, int pre_rows, int pre_per_wg
+
+// What a kernel instance of (NL, L, J, NWV, WPR) is made of.
+template <int NL, int L, int J, int NWV, int WPR>
+struct Q8Shape {
+    static constexpr int n = NL * 1024;
+    static constexpr int NG = NL * 64 / L;       // groups per row
+    static constexpr int THREADS = NWV * 64;
+    static constexpr int TEAMS = NWV / WPR;
+    static constexpr int SLOTS = TEAMS * J;      // rows per workgroup at most
+    static constexpr int NLW = NL / WPR;         // loads per wave and row
+    static constexpr int NGW = NLW * 64 / L;     // a wave's groups of a row
+    static constexpr int SK = (NGW + 63) / 64;   // scale loads per wave and row
+    static constexpr int IV = (n / 4 + THREADS - 1) / THREADS;  // input float4s per thread
+    static_assert(NWV % WPR == 0 && NL % WPR == 0 && NG % 4 == 0 && L <= 16, "wave layout");
+};
+
+// Issue the loads of this wave's scales and weight rows.
+template <class S, int J, int WPR>
+__device__ __forceinline__ void q8_issue_rows(const int8_t *w, const float *ws, int rows, int row0, int row_end, int wave,
+                                              int lane, float (&sc)[J][S::SK], u32x4 (&wv)[J][S::NLW])
 {
-    Q8Args a{};
-    a.x = pre_x;
-    a.rms_w = pre_rms_w;
-    a.w = pre_w;
-    a.ws = pre_ws;
-    a.rows = pre_rows;
-    constexpr int n = ACT * E;
-    constexpr int NG = ACT / L;            // groups per row
-    constexpr int VA = E / 4;              // input values per thread in the quantize step
-    constexpr int QT = n / VA;             // threads of the quantize step (4 * ACT)
-    constexpr int W = (L * E) / VA;        // threads per group in the quantize step (= 4 L)
-    constexpr int SLOTS = kQ8Teams * RPT;
-    static_assert(ACT <= kGemvThreads && ACT % L == 0 && ACT % 32 == 0 && NG % 4 == 0 && QT % W == 0,
-                  "thread layout");
+    const int team = wave / WPR, piece = wave % WPR;
+    const uint32_t w_bytes = (uint32_t)rows * (uint32_t)S::n, s_bytes = (uint32_t)rows * (S::NG * 4u);
+    const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(w, w_bytes);
+    const __amdgpu_buffer_rsrc_t s_rsrc = make_rsrc(ws, s_bytes);
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const int r = row0 + team + j * S::TEAMS;
+#pragma unroll
+        for (int k = 0; k < S::SK; k++) {
+            const int g = lane + 64 * k;  // of the wave's groups
+            const bool in = r < row_end && g < S::NGW;
+            const uint32_t off = (uint32_t)r * (S::NG * 4u) + 4u * (uint32_t)(piece * S::NGW + g);
+            sc[j][k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s_rsrc, (int)(in ? off : s_bytes), 0, kNt));
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const int r = row0 + team + j * S::TEAMS;
+        const uint32_t off = r < row_end ? (uint32_t)r * (uint32_t)S::n : w_bytes;
+#pragma unroll
+        for (int c = 0; c < S::NLW; c++)
+            wv[j][c] = __builtin_amdgcn_raw_buffer_load_b128(
+                w_rsrc, (int)(off + 16u * (uint32_t)lane + 1024u * (uint32_t)(piece * S::NLW + c)), 0, kNt);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int NL, int L, int J, int NWV, int WPR, int kIn, bool kResid>
+__global__ __launch_bounds__(NWV * 64) void q8_gemv_kernel(LEAP_Q8_PRELOAD_PARAMS, Q8Args args)
+{
+    using S = Q8Shape<NL, L, J, NWV, WPR>;
+    constexpr int n = S::n, NG = S::NG, IV = S::IV, THREADS = S::THREADS;
+    constexpr int W = 4 * L;  // threads per group in the quantize step
     __shared__ __align__(16) int8_t lds_xq[n];
     __shared__ float lds_xs[NG];
     // (float)idot and ws * sx of (row slot, group), [slot][group] with the
     // rows padded so that the chain lanes' 128-bit reads spread over the banks
     constexpr int NGP = NG + 4;
-    __shared__ __align__(16) float lds_f[SLOTS * NGP];
-    __shared__ __align__(16) float lds_c[SLOTS * NGP];
-    __shared__ float ss_part[kQ8Waves];
-    static_assert(2 * SLOTS * NGP * 4 + n + NG * 4 <= 64 * 1024, "LDS budget");
-    constexpr int SCL = (RPT * NG / 4 + kGemvThreads - 1) / kGemvThreads;  // scale float4s per thread
-    const int tid = threadIdx.x;
-    const int team = tid / kGemvThreads, tt = tid % kGemvThreads;
-    const int g = tt / L;  // this thread's group in the dot step
-    const int row0 = blockIdx.x * SLOTS;
-    const int rbase = row0 + team * RPT;
+    __shared__ __align__(16) float lds_f[S::SLOTS * NGP];
+    __shared__ __align__(16) float lds_c[S::SLOTS * NGP];
+    __shared__ float ss_part[NWV];
+    static_assert(2 * S::SLOTS * NGP * 4 + n + NG * 4 + NWV * 4 <= 64 * 1024, "LDS budget");
+    const int tid = threadIdx.x, lane = tid % 64;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int row0 = blockIdx.x * pre_per_wg;
+    const int row_end = min(row0 + pre_per_wg, pre_rows);
 
-    // 1. the input: E/4 fp32 values (and rms weights) per thread
-    float v[VA], gw[VA];
+    // 1. the input (and rms weights): float4s tid, tid + THREADS, ... (past n,
+    // zeros); then the rows
+    const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(pre_x, n * 4u);
+    const __amdgpu_buffer_rsrc_t g_rsrc = make_rsrc(pre_rms_w, n * 4u);
+    float4 v[IV], gw[IV];
 #pragma unroll
-    for (int e = 0; e < VA; e++) v[e] = gw[e] = 0.f;
-    if (QT < kQ8Threads && tid >= QT) {
-        // owns no input values
-    } else if constexpr (VA == 2) {
-        const float2 t = reinterpret_cast<const float2 *>(a.x)[tid];
-        v[0] = t.x;
-        v[1] = t.y;
-    } else {
-#pragma unroll
-        for (int c = 0; c < VA / 4; c++) {
-            const float4 t = reinterpret_cast<const float4 *>(a.x + tid * VA)[c];
-            v[4 * c] = t.x;
-            v[4 * c + 1] = t.y;
-            v[4 * c + 2] = t.z;
-            v[4 * c + 3] = t.w;
-        }
-    }
+    for (int i = 0; i < IV; i++) v[i] = buf_load4(x_rsrc, 16u * (uint32_t)(tid + i * THREADS));
     if constexpr (kIn == kQ8InRms) {
-        if (QT < kQ8Threads && tid >= QT) {
-        } else if constexpr (VA == 2) {
-            const float2 t = reinterpret_cast<const float2 *>(a.rms_w)[tid];
-            gw[0] = t.x;
-            gw[1] = t.y;
-        } else {
 #pragma unroll
-            for (int c = 0; c < VA / 4; c++) {
-                const float4 t = reinterpret_cast<const float4 *>(a.rms_w + tid * VA)[c];
-                gw[4 * c] = t.x;
-                gw[4 * c + 1] = t.y;
-                gw[4 * c + 2] = t.z;
-                gw[4 * c + 3] = t.w;
-            }
-        }
+        for (int i = 0; i < IV; i++) gw[i] = buf_load4(g_rsrc, 16u * (uint32_t)(tid + i * THREADS));
     }
     __builtin_amdgcn_sched_barrier(0);
+    float sc[J][S::SK];
+    u32x4 wv[J][S::NLW];
+    q8_issue_rows<S, J, WPR>(pre_w, pre_ws, pre_rows, row0, row_end, wave, lane, sc, wv);
 
-    // 2. this team's group scales (RPT * NG consecutive floats, as float4s),
-    // then its weight rows
-    gemv_f4 scv[SCL];
-#pragma unroll
-    for (int i = 0; i < SCL; i++) {
-        const int e = 4 * (tt + i * kGemvThreads);  // scale index in the team's block
-        const int r = min(rbase + e / NG, a.rows - 1);
-        if (e < RPT * NG)
-            scv[i] = __builtin_nontemporal_load(reinterpret_cast<const gemv_f4 *>(a.ws + (size_t)r * NG + e % NG));
-    }
-    Q8Row<E> wv[RPT];
-    if constexpr (ACT == kGemvThreads) {
-#pragma unroll
-        for (int j = 0; j < RPT; j++) {
-            const int r = min(rbase + j, a.rows - 1);
-            wv[j] = load_row_nt<E>(a.w + (size_t)r * n + tt * E);
-        }
-    } else {
-        const uint32_t w_bytes = (uint32_t)a.rows * (uint32_t)n;
-        const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(a.w, w_bytes);
-#pragma unroll
-        for (int j = 0; j < RPT; j++) {
-            const int r = min(rbase + j, a.rows - 1);
-            wv[j] = load_row_buf<E>(w_rsrc, tt < ACT ? (uint32_t)r * (uint32_t)n + (uint32_t)(tt * E) : w_bytes);
-        }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-
-    // 3. the input normalised (if asked) and quantized into LDS: group max
+    // 2. the input normalised (if asked) and quantized into LDS: group max
     // over W lanes, scale, round half away from zero
     if constexpr (kIn == kQ8InRms) {
         float ss = 0.f;
 #pragma unroll
-        for (int e = 0; e < VA; e++) ss += v[e] * v[e];
+        for (int i = 0; i < IV; i++) ss += dot4f(v[i], v[i]);
         ss = wave_sum(ss);
-        if (tid % 64 == 0) ss_part[tid / 64] = ss;
+        if (lane == 0) ss_part[wave] = ss;
         __syncthreads();
         ss = 0.f;
 #pragma unroll
-        for (int w = 0; w < kQ8Waves; w++) ss += ss_part[w];
+        for (int w = 0; w < NWV; w++) ss += ss_part[w];
         const float scale = 1.0f / sqrtf(ss / (float)n + 1e-5f);
 #pragma unroll
-        for (int e = 0; e < VA; e++) v[e] = gw[e] * (scale * v[e]);
+        for (int i = 0; i < IV; i++)
+            v[i] = make_float4(gw[i].x * (scale * v[i].x), gw[i].y * (scale * v[i].y), gw[i].z * (scale * v[i].z),
+                               gw[i].w * (scale * v[i].w));
     }
-    float m = 0.f;
 #pragma unroll
-    for (int e = 0; e < VA; e++) m = fmaxf(m, fabsf(v[e]));
-    m = group_max_w<W>(m);
-    const float sx = m * (1.0f / 127.0f);
-    const float id = sx != 0.0f ? __frcp_rn(sx) : 0.0f;
-    int8_t q[VA];
-#pragma unroll
-    for (int e = 0; e < VA; e++) q[e] = (int8_t)(int)roundf(v[e] * id);
-    if (QT < kQ8Threads && tid >= QT) {
-    } else if constexpr (VA == 2) {
-        *reinterpret_cast<short *>(lds_xq + tid * 2) = (short)((q[0] & 0xFF) | ((q[1] & 0xFF) << 8));
-    } else {
-#pragma unroll
-        for (int k = 0; k < VA / 4; k++)
-            reinterpret_cast<int *>(lds_xq + tid * VA)[k] =
-                (q[4 * k] & 0xFF) | ((q[4 * k + 1] & 0xFF) << 8) | ((q[4 * k + 2] & 0xFF) << 16) |
-                ((q[4 * k + 3] & 0xFF) << 24);
-    }
-    if (tid % W == 0 && tid < QT) lds_xs[tid / W] = sx;
-#pragma unroll
-    for (int i = 0; i < SCL; i++) {
-        const int e = 4 * (tt + i * kGemvThreads);
-        if (e < RPT * NG) {
-            float *dst = lds_c + (team * RPT + e / NG) * NGP + e % NG;
-            dst[0] = scv[i].x;
-            dst[1] = scv[i].y;
-            dst[2] = scv[i].z;
-            dst[3] = scv[i].w;
+    for (int i = 0; i < IV; i++) {
+        float m = fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w)));
+        m = group_max_w<W>(fmaxf(m, 0.f));  // (a group of NaNs: 0)
+        const float sx = m * (1.0f / 127.0f);
+        const float id = sx != 0.0f ? __frcp_rn(sx) : 0.0f;
+        auto q8 = [&](float t) { return (int)(int8_t)(int)roundf(t * id) & 0xFF; };
+        const int at = tid + i * THREADS;
+        if (n / 4 % THREADS == 0 || at < n / 4) {
+            reinterpret_cast<int *>(lds_xq)[at] = q8(v[i].x) | (q8(v[i].y) << 8) | (q8(v[i].z) << 16) | (q8(v[i].w) << 24);
+            if (at % W == 0) lds_xs[at / W] = sx;
         }
     }
     __syncthreads();
     // The outputs, from here on: the barriers above wait for every scalar
     // load in flight, and these are needed only at the end.
-    {
-        const Q8Args late = late_args(args, kQ8ArgsOffset);
-        a.out0 = late.out0;
-        a.out1 = late.out1;
-        a.out2 = late.out2;
-        a.n0 = late.n0;
-        a.n1 = late.n1;
-        a.xq_out = late.xq_out;
-        a.xs_out = late.xs_out;
-    }
+    const Q8Args a = late_args(args, kQ8ArgsOffset);
     if (blockIdx.x == 0 && a.xq_out) {  // the quantized input, for stage checks
-        for (int i = tid; i < n / 4; i += kQ8Threads)
+        for (int i = tid; i < n / 4; i += THREADS)
             reinterpret_cast<int *>(a.xq_out)[i] = reinterpret_cast<const int *>(lds_xq)[i];
-        for (int i = tid; i < NG; i += kQ8Threads) a.xs_out[i] = lds_xs[i];
+        for (int i = tid; i < NG; i += THREADS) a.xs_out[i] = lds_xs[i];
     }
 
-    // 4. exact group dot products, one (float, scale product) pair per group
-    const bool owns = ACT == kGemvThreads || tt < ACT;
-    int xq[E / 4];
+    // 3. exact group dot products, one (float, scale product) pair per group
+    const int team = wave / WPR, piece = wave % WPR;
 #pragma unroll
-    for (int k = 0; k < E / 4; k++) xq[k] = owns ? reinterpret_cast<const int *>(lds_xq + tt * E)[k] : 0;
-    const float sxg = owns ? lds_xs[g] : 0.f;
+    for (int k = 0; k < S::SK; k++) {
+        const int g = lane + 64 * k;
+        if (g < S::NGW) {
+            const float xs = lds_xs[piece * S::NGW + g];
 #pragma unroll
-    for (int j = 0; j < RPT; j++) {
-        int d = 0;
+            for (int j = 0; j < J; j++) lds_c[(team + j * S::TEAMS) * NGP + piece * S::NGW + g] = sc[j][k] * xs;
+        }
+    }
 #pragma unroll
-        for (int k = 0; k < E / 4; k++) d = __builtin_amdgcn_sdot4(xq[k], wv[j].v[k], d, false);
-        d = group_sum_i32<L>(d);
-        if (tt % L == 0 && owns) {
-            const int at = (team * RPT + j) * NGP + g;
-            lds_f[at] = (float)d;
-            lds_c[at] = lds_c[at] * sxg;
+    for (int c = 0; c < S::NLW; c++) {
+        const int at = piece * S::NLW + c;
+        const u32x4 xq = *reinterpret_cast<const u32x4 *>(lds_xq + 1024 * at + 16 * lane);
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            int d = __builtin_amdgcn_sdot4((int)xq.x, (int)wv[j][c].x, 0, false);
+            d = __builtin_amdgcn_sdot4((int)xq.y, (int)wv[j][c].y, d, false);
+            d = __builtin_amdgcn_sdot4((int)xq.z, (int)wv[j][c].z, d, false);
+            d = __builtin_amdgcn_sdot4((int)xq.w, (int)wv[j][c].w, d, false);
+            d = group_sum_i32<L>(d);
+            if (lane % L == 0) lds_f[(team + j * S::TEAMS) * NGP + at * (64 / L) + lane / L] = (float)d;
         }
     }
     __syncthreads();
 
-    // 5. the ordered accumulation, one lane per row
-    if (tid < SLOTS) {
+    // 4. the ordered accumulation, one lane per row
+    if (tid < row_end - row0) {
         float val = 0.f;
         const float4 *f4 = reinterpret_cast<const float4 *>(lds_f + tid * NGP);
         const float4 *c4 = reinterpret_cast<const float4 *>(lds_c + tid * NGP);
-        // The wo product's chain reads all its LDS pairs ahead (0.24 us at
-        // Llama-3-8B); the q/k/v product gains nothing and would spill.
-        constexpr int kChainUnroll = kIn == kQ8InF32 ? NG / 4 : 4;
+        // every LDS read ahead of the chain (0.05-0.3 us per launch against 4
+        // groups ahead); with 16 waves that would spill (Llama-3-70B q/k/v
+        // 17.2 -> 20.6 us)
+        constexpr int kChainUnroll = NWV >= 16 ? 8 : NG / 4;
 #pragma unroll kChainUnroll
         for (int j = 0; j < NG / 4; j++) {
             const float4 f = f4[j], c = c4[j];
@@ -386,69 +311,46 @@ __global__ __launch_bounds__(kQ8Threads) void q8_gemv_kernel(LEAP_Q8_PRELOAD_PAR
             val = __builtin_fmaf(f.w, c.w, val);
         }
         const int r = row0 + tid;
-        if (r < a.rows) {
-            if constexpr (kResid) {
-                a.out0[r] += val;
-            } else {
-                if (r < a.n0)
-                    a.out0[r] = val;
-                else if (r < a.n0 + a.n1)
-                    a.out1[r - a.n0] = val;
-                else
-                    a.out2[r - a.n0 - a.n1] = val;
-            }
+        if constexpr (kResid) {
+            a.out0[r] += val;
+        } else {
+            if (r < a.n0)
+                a.out0[r] = val;
+            else if (r < a.n0 + a.n1)
+                a.out1[r - a.n0] = val;
+            else
+                a.out2[r - a.n0 - a.n1] = val;
         }
     }
 }
 
 // The int8 weights alone (measurement only): the grid, block size, scale
-// loads and row loads of q8_gemv_kernel<E, L, RPT, ..., ACT> over w [rows][n]
-// and its scales ws [rows][n / gs], summed and kept only behind a test that
-// real data never meets.  The launch plus the bare weight stream of one
-// int8 projection.
-template <int E, int L, int RPT, int ACT = kGemvThreads>
-__global__ __launch_bounds__(kQ8Threads) void q8_floor_kernel(LEAP_Q8_PRELOAD_PARAMS, Q8Args a)
+// loads and row loads of q8_gemv_kernel<NL, L, J, NWV, WPR, ...> over w
+// [rows][n] and its scales ws [rows][n / gs], summed and kept only behind a
+// test that real data never meets.  The launch plus the bare weight stream of
+// one int8 projection.
+template <int NL, int L, int J, int NWV, int WPR>
+__global__ __launch_bounds__(NWV * 64) void q8_floor_kernel(LEAP_Q8_PRELOAD_PARAMS, Q8Args a)
 {
+    using S = Q8Shape<NL, L, J, NWV, WPR>;
     (void)pre_x;
     (void)pre_rms_w;
-    a.w = pre_w;
-    a.ws = pre_ws;
-    a.rows = pre_rows;
-    constexpr int n = ACT * E;
-    constexpr int NG = ACT / L;
-    constexpr int SLOTS = kQ8Teams * RPT;
-    constexpr int SCL = (RPT * NG / 4 + kGemvThreads - 1) / kGemvThreads;
     const int tid = threadIdx.x;
-    const int team = tid / kGemvThreads, tt = tid % kGemvThreads;
-    const int rbase = blockIdx.x * SLOTS + team * RPT;
-    gemv_f4 scv[SCL];
-#pragma unroll
-    for (int i = 0; i < SCL; i++) {
-        const int e = 4 * (tt + i * kGemvThreads);
-        const int r = min(rbase + e / NG, a.rows - 1);
-        scv[i] = e < RPT * NG ? __builtin_nontemporal_load(reinterpret_cast<const gemv_f4 *>(a.ws + (size_t)r * NG + e % NG))
-                              : gemv_f4{0.f, 0.f, 0.f, 0.f};
-    }
-    Q8Row<E> wv[RPT];
-    const uint32_t w_bytes = (uint32_t)a.rows * (uint32_t)n;
-    const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(a.w, w_bytes);
-#pragma unroll
-    for (int j = 0; j < RPT; j++) {
-        const int r = min(rbase + j, a.rows - 1);
-        if constexpr (ACT == kGemvThreads)
-            wv[j] = load_row_nt<E>(a.w + (size_t)r * n + tt * E);
-        else
-            wv[j] = load_row_buf<E>(w_rsrc, tt < ACT ? (uint32_t)r * (uint32_t)n + (uint32_t)(tt * E) : w_bytes);
-    }
-    int acc = 0;
-#pragma unroll
-    for (int j = 0; j < RPT; j++)
-#pragma unroll
-        for (int k = 0; k < E / 4; k++) acc ^= wv[j].v[k];
+    const int row0 = blockIdx.x * pre_per_wg;
+    float sc[J][S::SK];
+    u32x4 wv[J][S::NLW];
+    q8_issue_rows<S, J, WPR>(pre_w, pre_ws, pre_rows, row0, min(row0 + pre_per_wg, pre_rows),
+                             __builtin_amdgcn_readfirstlane(tid / 64), tid % 64, sc, wv);
+    unsigned acc = 0;
     float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < SCL; i++) s += (scv[i].x + scv[i].y) + (scv[i].z + scv[i].w);
-    if (acc == 0x7EADBEEF && __builtin_bit_cast(unsigned, s) == 0x7FC0DEADu) a.out0[tid] = s;
+    for (int j = 0; j < J; j++) {
+#pragma unroll
+        for (int c = 0; c < S::NLW; c++) acc ^= (wv[j][c].x ^ wv[j][c].y) ^ (wv[j][c].z ^ wv[j][c].w);
+#pragma unroll
+        for (int k = 0; k < S::SK; k++) s += sc[j][k];
+    }
+    if (acc == 0x7EADBEEFu && __builtin_bit_cast(unsigned, s) == 0x7FC0DEADu) a.out0[tid] = s;
 }
 
 }  // namespace leap

@@ -6,7 +6,7 @@
 //     kernels_decode_{64,128}f.hip: the flat kernels (batches) by head_dim;
 //   - kernels_gemv.hip: the fp32 projection GEMVs by model width;
 //   - kernels_q8.hip: the int8 W8A8 projection GEMVs by width, group size,
-//     rows per team and input kind.
+//     rows per workgroup and input kind.
 // leap_hip_attention.hip holds the host side and picks kernels through these
 // functions only.
 #pragma once
@@ -84,14 +84,19 @@ using GemvFloorFn = void (*)(const float *, int, float *);
 bool pick_proj(int dim, QkvFn *qkv, ProjFn *proj, int *rb, GemvFloorFn *floor = nullptr);
 
 // The int8 projections.
-// (x, rms_w, w, ws and rows preloaded, then leap::Q8Args)
-using Q8Fn = void (*)(const float *, const float *, const int8_t *, const float *, int, leap::Q8Args);
+// (x, rms_w, w, ws, rows and per_wg preloaded, then leap::Q8Args)
+using Q8Fn = void (*)(const float *, const float *, const int8_t *, const float *, int, int, leap::Q8Args);
+// A launch of an int8 projection: the kernel, the one with the same grid that
+// streams the weights alone (measurement), rows per workgroup and the grid.
+struct Q8Launch {
+    Q8Fn fn, floor;
+    int per_wg, grid, threads;
+};
 // True if (dim, gs) has int8 kernels.
 bool q8_supported(int dim, int gs);
-// The kernel of `kind` (leap::kQ8InRms or leap::kQ8InF32) for `rows` rows:
-// the smallest compiled rows-per-team count RPT with kQ8Teams * RPT * n_cu >=
-// rows, else the largest; *rpt receives it, and *floor (if not null) the
-// kernel with the same grid that streams the weights alone (measurement).
-Q8Fn pick_q8(int dim, int gs, int kind, int rows, int n_cu, int *rpt, Q8Fn *floor = nullptr);
+// The launch of `kind` (leap::kQ8InRms or leap::kQ8InF32) over `rows` rows:
+// the fewest workgroups per CU that the compiled sizes allow, of equally many
+// rows each, by the smallest such size; false for a shape without kernels.
+bool pick_q8(int dim, int gs, int kind, int rows, int n_cu, Q8Launch *out);
 
 }  // namespace leap_kernels

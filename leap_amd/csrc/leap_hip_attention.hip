@@ -681,12 +681,11 @@ int launch_block_q8(leap_hip_attention *h, int li, int layer, int pos, float *x,
     qa.n1 = kv;
     qa.xq_out = h->q8_act;
     qa.xs_out = h->q8_act_s;
-    int rpt = 0;
-    Q8Fn fn = pick_q8(dim, gs, leap::kQ8InRms, (int)rows_qkv, h->n_cu, &rpt);
-    if (!fn) return set_err(h, -EINVAL, "dim %d with group size %d has no int8 projection kernel", dim, gs);
-    int per_wg = leap::kQ8Teams * rpt;
-    HIP_TRY(h, launch_k(fn, dim3((unsigned)((rows_qkv + per_wg - 1) / per_wg)), dim3(leap::kQ8Threads), stream, qa.x,
-                        qa.rms_w, qa.w, qa.ws, qa.rows, qa));
+    Q8Launch l;
+    if (!pick_q8(dim, gs, leap::kQ8InRms, (int)rows_qkv, h->n_cu, &l))
+        return set_err(h, -EINVAL, "dim %d with group size %d has no int8 projection kernel", dim, gs);
+    HIP_TRY(h, launch_k(l.fn, dim3((unsigned)l.grid), dim3((unsigned)l.threads), stream, qa.x, qa.rms_w, qa.w, qa.ws,
+                        qa.rows, l.per_wg, qa));
     int8_t *aq = h->q8_act + dim;
     float *as = h->q8_act_s + dim / gs;
     if (int rc = launch(h, layer, 1, nullptr, pos, pos, pos + 1, q, k, v, xb, stream)) return rc;
@@ -699,11 +698,10 @@ int launch_block_q8(leap_hip_attention *h, int li, int layer, int pos, float *x,
     pa.n0 = dim;
     pa.xq_out = aq;
     pa.xs_out = as;
-    fn = pick_q8(dim, gs, leap::kQ8InF32, dim, h->n_cu, &rpt);
-    if (!fn) return set_err(h, -EINVAL, "dim %d with group size %d has no int8 projection kernel", dim, gs);
-    per_wg = leap::kQ8Teams * rpt;
-    HIP_TRY(h, launch_k(fn, dim3((unsigned)((dim + per_wg - 1) / per_wg)), dim3(leap::kQ8Threads), stream, pa.x,
-                        pa.rms_w, pa.w, pa.ws, pa.rows, pa));
+    if (!pick_q8(dim, gs, leap::kQ8InF32, dim, h->n_cu, &l))
+        return set_err(h, -EINVAL, "dim %d with group size %d has no int8 projection kernel", dim, gs);
+    HIP_TRY(h, launch_k(l.fn, dim3((unsigned)l.grid), dim3((unsigned)l.threads), stream, pa.x, pa.rms_w, pa.w, pa.ws,
+                        pa.rows, l.per_wg, pa));
     return 0;
 }
 
@@ -727,18 +725,16 @@ int launch_block_floor(leap_hip_attention *h, int layer, int pos, hipStream_t st
                                     kFloorStream))
                     return rc;
             const int rows = pass == 0 ? rows_qkv : dim;
-            int rpt = 0;
-            Q8Fn floor = nullptr;
-            if (!pick_q8(dim, gs, pass == 0 ? leap::kQ8InRms : leap::kQ8InF32, rows, h->n_cu, &rpt, &floor) || !floor)
+            Q8Launch l;
+            if (!pick_q8(dim, gs, pass == 0 ? leap::kQ8InRms : leap::kQ8InF32, rows, h->n_cu, &l))
                 return set_err(h, -EINVAL, "dim %d with group size %d has no int8 projection kernel", dim, gs);
             leap::Q8Args qa{};
             qa.w = pass == 0 ? h->w8_qkv + (size_t)li * rows_qkv * dim : h->w8_o + (size_t)li * dim * dim;
             qa.ws = pass == 0 ? h->s8_qkv + (size_t)li * rows_qkv * (dim / gs) : h->s8_o + (size_t)li * dim * (dim / gs);
             qa.rows = rows;
             qa.out0 = sink;
-            const int per_wg = leap::kQ8Teams * rpt;
-            HIP_TRY(h, launch_k(floor, dim3((unsigned)((rows + per_wg - 1) / per_wg)), dim3(leap::kQ8Threads), stream,
-                                qa.x, qa.rms_w, qa.w, qa.ws, qa.rows, qa));
+            HIP_TRY(h, launch_k(l.floor, dim3((unsigned)l.grid), dim3((unsigned)l.threads), stream, qa.x, qa.rms_w,
+                                qa.w, qa.ws, qa.rows, l.per_wg, qa));
         }
         return 0;
     }
@@ -800,7 +796,8 @@ int launch_block(leap_hip_attention *h, int layer, int pos, float *x, float *x_r
 // at the allocation-free step's set-up, so that no later launch allocates.
 hipError_t load_kernel_tables()
 {
-    int rpt = 0;
+    Q8Launch q8;
+    if (!pick_q8(4096, 64, leap::kQ8InRms, 6144, 256, &q8)) return hipErrorInvalidValue;
     const void *fns[] = {
         reinterpret_cast<const void *>(pick_kernel(64, 4, kDecode, false, false, false)),
         reinterpret_cast<const void *>(pick_kernel(64, 4, kDecode, false, true, false)),
@@ -809,7 +806,7 @@ hipError_t load_kernel_tables()
         reinterpret_cast<const void *>(pick_flat<64>(4, 0)),
         reinterpret_cast<const void *>(pick_flat<128>(4, 0)),
         reinterpret_cast<const void *>(pick_kernel(128, 4, kFloorLaunch, false, false, false)),
-        reinterpret_cast<const void *>(pick_q8(4096, 64, leap::kQ8InRms, 6144, 256, &rpt)),
+        reinterpret_cast<const void *>(q8.fn),
     };
     QkvFn qkv = nullptr;
     ProjFn proj = nullptr;
