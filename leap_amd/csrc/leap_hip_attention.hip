@@ -803,8 +803,6 @@ hipError_t load_kernel_tables()
         reinterpret_cast<const void *>(pick_kernel(64, 4, kDecode, false, true, false)),
         reinterpret_cast<const void *>(pick_kernel(128, 4, kDecode, false, false, false)),
         reinterpret_cast<const void *>(pick_kernel(128, 4, kDecode, false, true, false)),
-        reinterpret_cast<const void *>(pick_flat<64>(4, 0)),
-        reinterpret_cast<const void *>(pick_flat<128>(4, 0)),
         reinterpret_cast<const void *>(pick_kernel(128, 4, kFloorLaunch, false, false, false)),
         reinterpret_cast<const void *>(q8.fn),
     };
@@ -819,6 +817,12 @@ hipError_t load_kernel_tables()
     }
     hipFuncAttributes attr;
     return hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(qkv));
+}
+// The flat kernels' table, for a handle that can launch them.
+hipError_t load_flat_table(int head_dim)
+{
+    hipFuncAttributes attr;
+    return hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(head_dim == 64 ? pick_flat<64>(4, 0) : pick_flat<128>(4, 0)));
 }
 
 // Run the XCC probe over n_wg workgroups of the decode kernel's block size
@@ -959,7 +963,10 @@ int leap_hip_attention_create(const leap_hip_attention_config *cfg, leap_hip_att
     // (and a flat launch's: records per XCD for its workgroups and at most
     // kFlatMaxItems groups)
     const int items = (int)std::min<size_t>((n_pg + leap::kXcds - 1) / leap::kXcds, leap::kFlatMaxItems);
-    if (items >= 2) h->max_flat = kFlatPerCu * h->n_cu / leap::kXcds;
+    if (items >= 2) {
+        h->max_flat = kFlatPerCu * h->n_cu / leap::kXcds;
+        CREATE_TRY(load_flat_table(c.head_dim));
+    }
     const size_t ws_rows = std::max(n_pg * kvv.group * leap::records_per_head(h->max_chunks),
                                     (size_t)leap::kXcds * kvv.group * leap::flat_records(h->max_flat, items));
     CREATE_TRY(hipMalloc(&h->ws_o, ws_rows * c.head_dim * sizeof(float)));
