@@ -74,14 +74,22 @@ extern template KernelFn pick_flat<128>(int, int);
 // The cross-XCD merge of a spread launch.
 MergeFn pick_merge(int hd, int g);
 
-// The fp32 projections by dim = 1024 * NC: *rb rows per workgroup.
+// The fp32 projections.
 // (the fields of leap::QkvArgs and leap::ProjArgs as scalar arguments, which
 // the dispatch preloads)
 using QkvFn = void (*)(const float *, const float *, const float *, float *, float *, float *, int, int);
 using ProjFn = void (*)(const float *, const float *, float *, int);
 // (w, rows, sink): the same grid streaming the weights alone (measurement)
 using GemvFloorFn = void (*)(const float *, int, float *);
-bool pick_proj(int dim, QkvFn *qkv, ProjFn *proj, int *rb, GemvFloorFn *floor = nullptr);
+// A launch over `rows` rows of width dim: the q/k/v kernel, the wo kernel, the
+// floor and their grid; false for a width without kernels.
+struct ProjLaunch {
+    QkvFn qkv;
+    ProjFn proj;
+    GemvFloorFn floor;
+    int grid;
+};
+bool pick_proj(int dim, int rows, int n_cu, ProjLaunch *out);
 
 // The int8 projections.
 // (x, rms_w, w, ws, rows and per_wg preloaded, then leap::Q8Args)

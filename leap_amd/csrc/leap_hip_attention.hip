@@ -738,17 +738,14 @@ int launch_block_floor(leap_hip_attention *h, int layer, int pos, hipStream_t st
         }
         return 0;
     }
-    QkvFn qkv;
-    ProjFn proj;
-    GemvFloorFn floor = nullptr;
-    int rb;
-    if (!pick_proj(dim, &qkv, &proj, &rb, &floor))
+    ProjLaunch qkv, proj;
+    if (!pick_proj(dim, rows_qkv, h->n_cu, &qkv) || !pick_proj(dim, dim, h->n_cu, &proj))
         return set_err(h, -EINVAL, "dim %d: the projections need dim in {2048, 3072, 4096, 5120, 8192}", dim);
-    HIP_TRY(h, launch_k(floor, dim3((unsigned)((rows_qkv + rb - 1) / rb)), dim3(leap::kGemvThreads), stream,
+    HIP_TRY(h, launch_k(qkv.floor, dim3((unsigned)qkv.grid), dim3(leap::kGemvThreads), stream,
                         (const float *)(h->w_qkv + (size_t)li * rows_qkv * dim), rows_qkv, sink));
     if (int rc = launch(h, layer, 1, nullptr, pos, pos, pos + 1, nullptr, nullptr, nullptr, sink, stream, kFloorStream))
         return rc;
-    HIP_TRY(h, launch_k(floor, dim3((unsigned)((dim + rb - 1) / rb)), dim3(leap::kGemvThreads), stream,
+    HIP_TRY(h, launch_k(proj.floor, dim3((unsigned)proj.grid), dim3(leap::kGemvThreads), stream,
                         (const float *)(h->w_o + (size_t)li * dim * dim), dim, sink));
     return 0;
 }
@@ -760,11 +757,9 @@ int launch_block(leap_hip_attention *h, int layer, int pos, float *x, float *x_r
     const int li = layer - h->cfg.layer_begin;
     if (h->w_fmt == 0 || !h->w_set[li]) return set_err(h, -EINVAL, "no weights set for layer %d", layer);
     if (h->w_fmt == 2) return launch_block_q8(h, li, layer, pos, x, x_res, stream);
-    QkvFn qkv;
-    ProjFn proj;
-    int rb;
     const int dim = h->q_dim, kv = h->kv_dim;
-    if (!pick_proj(dim, &qkv, &proj, &rb))
+    ProjLaunch qkv, proj;
+    if (!pick_proj(dim, dim + 2 * kv, h->n_cu, &qkv) || !pick_proj(dim, dim, h->n_cu, &proj))
         return set_err(h, -EINVAL, "dim %d: the projections need dim in {2048, 3072, 4096, 5120, 8192}", dim);
     float *q = h->blk, *k = q + dim, *v = k + kv, *xb = v + kv;
     leap::QkvArgs qa{};
@@ -776,16 +771,16 @@ int launch_block(leap_hip_attention *h, int layer, int pos, float *x, float *x_r
     qa.v = v;
     qa.dim = dim;
     qa.kv_dim = kv;
-    HIP_TRY(h, launch_k(qkv, dim3((unsigned)((dim + 2 * kv + rb - 1) / rb)), dim3(leap::kGemvThreads), stream, qa.x,
-                        qa.rms_w, qa.w, qa.q, qa.k, qa.v, qa.dim, qa.kv_dim));
+    HIP_TRY(h, launch_k(qkv.qkv, dim3((unsigned)qkv.grid), dim3(leap::kGemvThreads), stream, qa.x, qa.rms_w, qa.w,
+                        qa.q, qa.k, qa.v, qa.dim, qa.kv_dim));
     if (int rc = launch(h, layer, 1, nullptr, pos, pos, pos + 1, q, k, v, xb, stream)) return rc;
     leap::ProjArgs pa{};
     pa.xb = xb;
     pa.w = h->w_o + (size_t)li * dim * dim;
     pa.x = x_res;
     pa.d = dim;
-    HIP_TRY(h, launch_k(proj, dim3((unsigned)((dim + rb - 1) / rb)), dim3(leap::kGemvThreads), stream, pa.xb, pa.w,
-                        pa.x, pa.d));
+    HIP_TRY(h, launch_k(proj.proj, dim3((unsigned)proj.grid), dim3(leap::kGemvThreads), stream, pa.xb, pa.w, pa.x,
+                        pa.d));
     return 0;
 }
 
@@ -806,17 +801,15 @@ hipError_t load_kernel_tables()
         reinterpret_cast<const void *>(pick_kernel(128, 4, kFloorLaunch, false, false, false)),
         reinterpret_cast<const void *>(q8.fn),
     };
-    QkvFn qkv = nullptr;
-    ProjFn proj = nullptr;
-    int rb = 0;
-    pick_proj(4096, &qkv, &proj, &rb);
+    ProjLaunch proj;
+    if (!pick_proj(4096, 4096, 256, &proj)) return hipErrorInvalidValue;
     for (const void *f : fns) {
         hipFuncAttributes attr;
         if (!f) return hipErrorInvalidValue;
         if (hipError_t e = hipFuncGetAttributes(&attr, f); e != hipSuccess) return e;
     }
     hipFuncAttributes attr;
-    return hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(qkv));
+    return hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(proj.proj));
 }
 // The flat kernels' table, for a handle that can launch them.
 hipError_t load_flat_table(int head_dim)
@@ -1292,11 +1285,9 @@ int leap_hip_attention_set_layer_weights(leap_hip_attention *h, int layer, const
     if (!h) return -EINVAL;
     if (int rc = check_layer(h, layer)) return rc;
     if (!rms_att || !wq || !wk || !wv || !wo) return set_err(h, -EINVAL, "NULL weight");
-    QkvFn qkv;
-    ProjFn proj;
-    int rb;
     const int dim = h->q_dim, kv = h->kv_dim;
-    if (!pick_proj(dim, &qkv, &proj, &rb))
+    ProjLaunch proj;
+    if (!pick_proj(dim, dim, h->n_cu, &proj))
         return set_err(h, -EINVAL, "dim %d: the projections need dim in {2048, 3072, 4096, 5120, 8192}", dim);
     if (h->w_fmt == 2) return set_err(h, -EINVAL, "this handle holds int8 weights");
     HIP_TRY(h, hipSetDevice(h->cfg.device));
