@@ -454,14 +454,17 @@ __device__ __forceinline__ void buf_store2(__amdgpu_buffer_rsrc_t r, uint32_t of
 // ---- wave helpers ---------------------------------------------------------
 //
 // The q.K scores come out of 4x4x1 MFMAs with lane = 32*kq + 4*ksl + kj
-// holding the partial dot product of K row 4*kq + kj over dim slice ksl
-// (eight slices).  The slices are summed with DPP inside each 16-lane row
-// (row_ror by 4 and by 8 lanes add the lanes of equal kj) and then across the
-// row pair with v_permlane16_swap, which hands row 0 to row 1 and row 2 to
-// row 3: rows 1 and 3 (lanes 16-31 and 48-63) end up holding the finished
-// scores, rows 0 and 2 hold nothing useful.  The wave max / sum over those
-// rows takes the quad (kj) with DPP and the two rows with v_readlane, which
-// leaves a wave-uniform result.
+// holding the partial dot product of K row 4*kq + kj of an 8-row set over dim
+// slice ksl (eight slices).  The slices are summed with DPP inside each 16-lane
+// row (row_ror by 4 and by 8 lanes add the lanes of equal kj) and then across
+// the row pair, for the sub-tile's two 8-row sets at once: v_permlane16_swap
+// hands the odd rows of the first set's register and the even rows of the
+// second's to each other, and one addition leaves the first set's scores in
+// rows 0 and 2 and the second's in rows 1 and 3 (slice_sum2).  One register
+// then holds the 16 rows of the sub-tile (score_row: the lane's row), each in
+// four lanes, and the softmax works on half the registers that one set each
+// would take.  The wave max / sum takes the quad (kj) with DPP and the four
+// rows with v_readlane, which leaves a wave-uniform result.
 
 template <int CTRL>
 __device__ __forceinline__ float dpp(float x)
@@ -475,21 +478,20 @@ __device__ __forceinline__ float lane_value(float x, int lane)
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
 }
 
-// Odd 16-lane rows receive the even row before them (the first result of
-// v_permlane16_swap with both operands x; the second result is not used).
-__device__ __forceinline__ float from_even_row(float x)
-{
-    const unsigned u = __builtin_bit_cast(unsigned, x);
-    return __builtin_bit_cast(float, __builtin_amdgcn_permlane16_swap(u, u, false, false)[0]);
-}
-
-// Sum of the eight dim slices of a score: valid in rows 1 and 3.
-__device__ __forceinline__ float slice_sum(float x)
+// Sums of the eight dim slices of two row sets' scores: x's in the even
+// 16-lane rows, y's in the odd ones.
+__device__ __forceinline__ float slice_sum2(float x, float y)
 {
     x += dpp<0x124>(x);  // row_ror:4
+    y += dpp<0x124>(y);
     x += dpp<0x128>(x);  // row_ror:8
-    return x + from_even_row(x);
+    y += dpp<0x128>(y);
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, y),
+                                                    false, false);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
 }
+// The sub-tile row whose score slice_sum2 leaves in a lane.
+__device__ __forceinline__ int score_row(int lane) { return 8 * ((lane >> 4) & 1) + 4 * (lane >> 5) + (lane & 3); }
 
 // Max / sum over R rows of 16 lanes (R = 1, 2 or 4): rows 2k and 2k + 1
 // meet, then the two halves of the wave, through the lane crossbar
@@ -507,20 +509,20 @@ __device__ __forceinline__ float rows_reduce(float x)
     return x;
 }
 
-// Max / sum over the score lanes (rows 1 and 3) of a value that is uniform
-// across the eight slice lanes of each K row; wave-uniform result.
+// Max / sum over a sub-tile's rows of a value that is uniform across the four
+// lanes of each row; wave-uniform result.
 __device__ __forceinline__ float score_rows_max(float x)
 {
     x = fmaxf(x, dpp<0xB1>(x));  // quad_perm [1,0,3,2]
     x = fmaxf(x, dpp<0x4E>(x));  // quad_perm [2,3,0,1]
-    return fmaxf(lane_value(x, 16), lane_value(x, 48));
+    return fmaxf(fmaxf(lane_value(x, 0), lane_value(x, 16)), fmaxf(lane_value(x, 32), lane_value(x, 48)));
 }
 
 __device__ __forceinline__ float score_rows_sum(float x)
 {
     x += dpp<0xB1>(x);
     x += dpp<0x4E>(x);
-    return lane_value(x, 16) + lane_value(x, 48);
+    return (lane_value(x, 0) + lane_value(x, 16)) + (lane_value(x, 32) + lane_value(x, 48));
 }
 
 // acc += a[c] * b[c] for the four float4 components, one 4x4x1 MFMA each:
@@ -582,6 +584,8 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // Growth of the running max (log2 units) tolerated before the accumulators
 // are rescaled: p = 2^(s - m_ref) stays below 2^kLazyMax.
 constexpr float kLazyMax = 8.0f;
+// The reference max before any score: the lowest finite value.
+constexpr float kLowest = -3.402823466e+38f;
 
 template <int HD, int G, int NW>
 struct Shape {
@@ -599,7 +603,7 @@ struct Shape {
     static constexpr int GM = G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : 8;
     static constexpr int MG = THREADS / (GM * D4);
     static_assert(HD % 32 == 0, "head_dim vs K slices");
-    static_assert(R % 8 == 0 && R % RPV == 0, "sub-tile shape");
+    static_assert(KS == 2 && R % RPV == 0, "sub-tile shape");
     static_assert(G <= 8, "q heads per KV head");
     static_assert(MG >= 1 && THREADS % (GM * D4) == 0, "merge layout");
 };
@@ -810,7 +814,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     // dim; the eight slices are summed afterwards (slice_sum).
     const int kj = lane & 3, ksl = (lane >> 2) & 7, kq = lane >> 5;
     const int krow = 4 * kq + kj;
-    const bool score_lane = (lane >> 4) & 1;  // rows 1 and 3 of the wave
+    const int srow = score_row(lane);  // the row whose score this lane holds
     // V layout: lane = vg*LPV + vj; lane holds dims 4*vj .. +3.
     const int vg = lane / LPV, vj = lane % LPV;
 
@@ -936,7 +940,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     f32x4 acc[GQ][4];
 #pragma unroll
     for (int h = 0; h < G; h++) {
-        m_ref[h] = -INFINITY;
+        m_ref[h] = kLowest;
         l_run[h] = 0.0f;
     }
 #pragma unroll
@@ -945,18 +949,14 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
         for (int e = 0; e < 4; e++) acc[q][e] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // FLAT: this wave's outputs so far, relative to 2^m_sum, as its partials in
-    // the combine buffer (m_sum: -inf before the first)
+    // the combine buffer
     float m_sum[FLAT ? G : 1];
-    if constexpr (FLAT) {
-#pragma unroll
-        for (int h = 0; h < G; h++) m_sum[h] = -INFINITY;
-    }
     bool flushed = false;
     auto flush = [&]() {
 #pragma unroll
         for (int h = 0; h < G; h++) {
             float4 o = make_float4(acc[h / 4][0][h % 4], acc[h / 4][1][h % 4], acc[h / 4][2][h % 4], acc[h / 4][3][h % 4]);
-            if (flushed) fma4(o, m_sum[h] == -INFINITY ? 0.0f : fast_exp2(m_sum[h] - m_ref[h]), comb_o[wave][vg][h][vj]);
+            if (flushed) fma4(o, fast_exp2(m_sum[h] - m_ref[h]), comb_o[wave][vg][h][vj]);
             comb_o[wave][vg][h][vj] = o;
             m_sum[h] = m_ref[h];
         }
@@ -1007,110 +1007,104 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
             // 32*f + 4*ksl .. +3 of k_new and of the table row
             if (lane < D4) nt_lds[lane] = knew_l;
             __builtin_amdgcn_wave_barrier();
-            float4 knew[NF], tab[NF];
+            // (one column at a time: the loop's registers are all live here)
 #pragma unroll
             for (int f = 0; f < NF; f++) {
-                knew[f] = nt_lds[8 * f + ksl];
-                tab[f] = nt_lds[D4 + 8 * f + ksl];
-            }
+                const float4 knew = rope4(nt_lds[8 * f + ksl], nt_lds[D4 + 8 * f + ksl]);
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                const int t = base + ks * 8 + krow;
-                if (t == pos) {
-#pragma unroll
-                    for (int f = 0; f < NF; f++) {
-                        kb[ks][f] = rope4(knew[f], tab[f]);
-                        if (store_new)
-                            *reinterpret_cast<float4 *>(kc + (size_t)t * kv_dim + 4 * (8 * f + ksl)) = kb[ks][f];
+                for (int ks = 0; ks < KS; ks++) {
+                    const int t = base + ks * 8 + krow;
+                    if (t == pos) {
+                        kb[ks][f] = knew;
+                        if (store_new) *reinterpret_cast<float4 *>(kc + (size_t)t * kv_dim + 4 * (8 * f + ksl)) = knew;
                     }
                 }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
 
-        // Scores (log2 units) on the matrix cores: s[ks][h] is head h at row
-        // ks*8 + krow in the score lanes, -inf elsewhere and past pos.
-        float s[KS][G];
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const bool ok = score_lane && (base + ks * 8 + krow <= last);
+        // Scores (log2 units) on the matrix cores: s[h] is head h at row srow
+        // of the sub-tile, -inf past pos.
+        float s[G];
+        {
+            const bool ok = base + srow <= last;
 #pragma unroll
             for (int qd = 0; qd < GQ; qd++) {
-                f32x4 d = {0.f, 0.f, 0.f, 0.f};
-                if constexpr (MFMA) {
+                f32x4 d[KS];
 #pragma unroll
-                    for (int f = 0; f < NF; f++) d = mfma4(qa[qd][f], kb[ks][f], d);
-                } else {
-                    // lane (kq, ksl, kj): head 4*qd + i times row 4*kq + kj over
-                    // this lane's dims, the partial the MFMA leaves in d[i]
+                for (int ks = 0; ks < KS; ks++) {
+                    d[ks] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    if constexpr (MFMA) {
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        if (4 * qd + i >= G) continue;
+                        for (int f = 0; f < NF; f++) d[ks] = mfma4(qa[qd][f], kb[ks][f], d[ks]);
+                    } else {
+                        // lane (kq, ksl, kj): head 4*qd + i times row 4*kq + kj
+                        // over this lane's dims, the partial the MFMA leaves in
+                        // d[i]
 #pragma unroll
-                        for (int f = 0; f < NF; f++) {
-                            const float4 qv = q_lds[4 * qd + i][8 * f + ksl];
-                            d[i] += qv.x * kb[ks][f].x + qv.y * kb[ks][f].y + qv.z * kb[ks][f].z + qv.w * kb[ks][f].w;
+                        for (int i = 0; i < 4; i++) {
+                            if (4 * qd + i >= G) continue;
+#pragma unroll
+                            for (int f = 0; f < NF; f++) {
+                                const float4 qv = q_lds[4 * qd + i][8 * f + ksl];
+                                d[ks][i] += qv.x * kb[ks][f].x + qv.y * kb[ks][f].y + qv.z * kb[ks][f].z + qv.w * kb[ks][f].w;
+                            }
                         }
                     }
                 }
+                // cross-lane: every lane takes part
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     if (4 * qd + i >= G) continue;
-                    const float v = slice_sum(d[i]);  // cross-lane: every lane takes part
-                    s[ks][4 * qd + i] = ok ? v : -INFINITY;
+                    const float v = slice_sum2(d[0][i], d[1][i]);
+                    s[4 * qd + i] = ok ? v : -INFINITY;
                 }
             }
         }
 
         // Online softmax with a lazily raised reference max: only when some
         // score exceeds m_ref + kLazyMax is the wave max taken and the
-        // accumulators rescaled (always on the first valid tile).
-        float mt[G];
-        bool grow = false;
+        // accumulators rescaled (always on the first tile with a valid row:
+        // m_ref starts at the lowest finite value, from which any other
+        // finite score is further away than kLazyMax).  A masked score is
+        // -inf, and 2^(-inf - m_ref) is 0.
+        float t[G], over = -INFINITY;
 #pragma unroll
         for (int h = 0; h < G; h++) {
-            mt[h] = s[0][h];
-#pragma unroll
-            for (int ks = 1; ks < KS; ks++) mt[h] = fmaxf(mt[h], s[ks][h]);
-            grow |= mt[h] > m_ref[h] + kLazyMax;
+            t[h] = s[h] - m_ref[h];
+            over = fmaxf(over, t[h]);
         }
         if (i == 0) tl.mark(kTlScored);
-        if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+        if (__builtin_amdgcn_ballot_w64(over > kLazyMax) != 0) {
 #pragma unroll
             for (int h = 0; h < G; h++) {
-                const float m_new = fmaxf(m_ref[h], score_rows_max(mt[h]));
-                const float alpha = (m_ref[h] == -INFINITY) ? 0.0f : fast_exp2(m_ref[h] - m_new);
+                const float m_new = fmaxf(m_ref[h], score_rows_max(s[h]));
+                const float alpha = fast_exp2(m_ref[h] - m_new);
 #pragma unroll
                 for (int e = 0; e < 4; e++) acc[h / 4][e][h % 4] *= alpha;
                 l_run[h] *= alpha;
                 m_ref[h] = m_new;
+                t[h] = s[h] - m_new;
             }
         }
+        // (the four lanes of a row hold the same p: l is kept per lane and
+        // summed over the rows once at the end)
 #pragma unroll
         for (int h = 0; h < G; h++) {
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                s[ks][h] = (s[ks][h] == -INFINITY) ? 0.0f : fast_exp2(s[ks][h] - m_ref[h]);
-                // the eight slice lanes of a row hold the same p: l is kept
-                // per lane and summed over the score rows once at the end
-                l_run[h] += s[ks][h];
-            }
+            s[h] = fast_exp2(t[h]);
+            l_run[h] += s[h];
         }
 
-        // Probabilities to LDS, [row][head], from one slice lane per row
-        // (lanes 16-19 and 48-51).
-        if ((lane & 0x1C) == 0x10) {
+        // Probabilities to LDS, [row][head], from one lane per row.
+        if ((lane & 0xC) == 0) {
+            float *dst = &p_lds[wave][srow * G];
+            if constexpr (G % 4 == 0) {
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                float *dst = &p_lds[wave][(ks * 8 + krow) * G];
-                if constexpr (G % 4 == 0) {
+                for (int qd = 0; qd < GQ; qd++)
+                    reinterpret_cast<float4 *>(dst)[qd] = make_float4(s[4 * qd], s[4 * qd + 1], s[4 * qd + 2], s[4 * qd + 3]);
+            } else {
 #pragma unroll
-                    for (int qd = 0; qd < GQ; qd++)
-                        reinterpret_cast<float4 *>(dst)[qd] =
-                            make_float4(s[ks][4 * qd], s[ks][4 * qd + 1], s[ks][4 * qd + 2], s[ks][4 * qd + 3]);
-                } else {
-#pragma unroll
-                    for (int h = 0; h < G; h++) dst[h] = s[ks][h];
-                }
+                for (int h = 0; h < G; h++) dst[h] = s[h];
             }
         }
         __builtin_amdgcn_wave_barrier();
@@ -1166,7 +1160,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     // combine buffer), scores it against each head (a dot product per lane,
     // summed over the 16-lane rows with DPP and over the rows with
     // v_readlane: wave-uniform), and adds p = 2^(s - m_ref) and p * v_new to
-    // the head's sum (lane 16's share of it, as score_rows_sum reads) and
+    // the head's sum (lane 0's share of it, as score_rows_sum reads) and
     // accumulators (lanes vg == 0: V row slot 0 of dims 4*vj .. +3), raising
     // the reference max first if the score exceeds it by kLazyMax.  The
     // heads' chains are independent and laid out step by step, so that they
@@ -1215,7 +1209,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
 #pragma unroll
                 for (int h = 0; h < G; h++) {
                     const float m_new = fmaxf(m_ref[h], sh[h]);
-                    const float alpha = (m_ref[h] == -INFINITY) ? 0.0f : fast_exp2(m_ref[h] - m_new);
+                    const float alpha = fast_exp2(m_ref[h] - m_new);
 #pragma unroll
                     for (int e = 0; e < 4; e++) acc[h / 4][e][h % 4] *= alpha;
                     l_run[h] *= alpha;
@@ -1225,7 +1219,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
 #pragma unroll
             for (int h = 0; h < G; h++) {
                 const float p = fast_exp2(sh[h] - m_ref[h]);
-                l_run[h] += (lane == 16) ? p : 0.0f;
+                l_run[h] += (lane == 0) ? p : 0.0f;
                 const float pv = (vg == 0) ? p : 0.0f;
                 acc[h / 4][0][h % 4] += pv * vnew_l.x;
                 acc[h / 4][1][h % 4] += pv * vnew_l.y;
