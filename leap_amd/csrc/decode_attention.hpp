@@ -579,6 +579,22 @@ __device__ __forceinline__ float4 rope4(float4 x, float4 t)
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// One register of two: the lower half of the lanes gets the sum of x's two
+// halves, the upper half the sum of y's.
+__device__ __forceinline__ float halves_sum2(float x, float y)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, y),
+                                                    false, false);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+// The same within each pair of 16-lane rows.
+__device__ __forceinline__ float rows_sum2(float x, float y)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, y),
+                                                    false, false);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+
 // ---- the fused decode-attention kernel --------------------------------------
 
 // Growth of the running max (log2 units) tolerated before the accumulators
@@ -607,6 +623,41 @@ struct Shape {
     static_assert(G <= 8, "q heads per KV head");
     static_assert(MG >= 1 && THREADS % (GM * D4) == 0, "merge layout");
 };
+
+// The sums of a wave's output accumulators over its V row slots (lanes of
+// equal dims: the halves of the wave at head_dim 128, its four 16-lane rows at
+// 64), put(first, head, dims 4*vj .. +3) in one lane per (head, column); first
+// is the lowest head of that register, a constant once unrolled.  The swaps
+// that bring two registers' slots together leave one head per half (row), so
+// that a quad of heads takes two (one) 16-byte writes per lane to LDS in place
+// of four, and the waves' combine reads half (a quarter) of the bytes.
+template <int HD, int G, class Put>
+__device__ __forceinline__ void slot_sums(const f32x4 (&acc)[(G + 3) / 4][4], int lane, Put put)
+{
+#pragma unroll
+    for (int q = 0; q < (G + 3) / 4; q++) {
+        // head 4q + i's component e; zero past the heads
+        auto at = [&](int i, int e) { return 4 * q + i < G ? acc[q][e][i] : 0.0f; };
+        if constexpr (HD == 128) {
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {
+                if (4 * q + i >= G) continue;
+                const int h = 4 * q + i + (lane >> 5);
+                const float4 o = make_float4(halves_sum2(at(i, 0), at(i + 1, 0)), halves_sum2(at(i, 1), at(i + 1, 1)),
+                                             halves_sum2(at(i, 2), at(i + 1, 2)), halves_sum2(at(i, 3), at(i + 1, 3)));
+                if (h < G) put(4 * q + i, h, o);
+            }
+        } else {
+            // rows 0-3 of the wave: heads 0, 1, 2, 3 of the quad
+            const int h = 4 * q + (lane >> 4);
+            float c[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                c[e] = halves_sum2(rows_sum2(at(0, e), at(1, e)), rows_sum2(at(2, e), at(3, e)));
+            if (h < G) put(4 * q, h, make_float4(c[0], c[1], c[2], c[3]));
+        }
+    }
+}
 
 // MFMA: the score and weighted-V products on the matrix cores (4x4x1 f32
 // MFMAs); false: the same products as per-lane VALU FMAs, leaving the same
@@ -758,7 +809,9 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     // (what follows from the thread's number is worked out again for each
     // segment: held through the ones before, it took 256 registers and scratch)
     if constexpr (FLAT) asm volatile("" : "+v"(tid));
-    const int wave = tid / kWave;
+    // (scalar with PART, whose tests of the wave's rows it makes scalar too; in
+    // the whole-pass instances it measured 0.5-1% slower at ctx 2048-4096)
+    const int wave = PART ? __builtin_amdgcn_readfirstlane(tid / kWave) : tid / kWave;
     const int lane = tid % kWave;
 
     const int T = pos + 1;
@@ -797,7 +850,17 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
 
     __shared__ __align__(16) float p_lds[NW][R * G];
     __shared__ float4 q_lds[G][HD / 4];  // rotated, scaled q of the group's heads
-    __shared__ float4 comb_o[NW][RPV][G][D4];
+    // The waves' partial outputs, [wave][V row slot][head][column]; also staging
+    // for the new token (per wave) and the merge's scratch.  With PART a wave
+    // sums its slots first (slot_sums): same process, graph replay, Llama-3-8B
+    // heads ctx 256 5.10 -> 4.95 us, TinyLlama ctx 64 3.56 -> 3.48, and in flat
+    // launches a quarter to half the bytes of every flush.  Whole-pass launches
+    // keep the slots apart: the sums' extra steps made Llama-3-8B ctx 4096
+    // 0.8% slower.
+    constexpr int SLOTS = PART ? 1 : RPV;
+    // (a float4 per lane and wave at least, for the staging and the merge)
+    constexpr int CSLOTS = SLOTS * G * D4 < kWave ? (kWave + G * D4 - 1) / (G * D4) : SLOTS;
+    __shared__ float4 comb_o[NW][CSLOTS][G][D4];
     __shared__ __align__(16) float comb_l[G][NW];  // [head][wave]: a head's NW values in one read
     __shared__ __align__(16) float comb_m[G][NW];
     // FLAT: the new token's staging, apart from the combine buffer, which holds
@@ -920,7 +983,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     // (unused until the waves combine): float4 [D4, 2*D4); the k_new row
     // goes to [0, D4) when it is needed.
     float4 *nt_lds = FLAT ? &stage_lds[FLAT ? wave : 0][0] : &comb_o[wave][0][0][0];
-    static_assert(RPV * G >= 2, "new-token staging");
+    static_assert(CSLOTS * G >= 2, "new-token staging");
     if (lane < HD / 2) reinterpret_cast<float2 *>(nt_lds + D4)[lane] = qt[0];
     __syncthreads();
     tl.mark(kTlPrologue);
@@ -953,13 +1016,23 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     float m_sum[FLAT ? G : 1];
     bool flushed = false;
     auto flush = [&]() {
+        float ratio[G];  // from the sums' reference max to the current one
 #pragma unroll
         for (int h = 0; h < G; h++) {
-            float4 o = make_float4(acc[h / 4][0][h % 4], acc[h / 4][1][h % 4], acc[h / 4][2][h % 4], acc[h / 4][3][h % 4]);
-            if (flushed) fma4(o, fast_exp2(m_sum[h] - m_ref[h]), comb_o[wave][vg][h][vj]);
-            comb_o[wave][vg][h][vj] = o;
+            ratio[h] = fast_exp2(m_sum[h] - m_ref[h]);
             m_sum[h] = m_ref[h];
         }
+        slot_sums<HD, G>(acc, lane, [&](int h0, int h, float4 o) {
+            float4 *dst = &comb_o[wave][0][h][vj];
+            if (flushed) {
+                auto of = [&](int j) { return ratio[h0 + j < G ? h0 + j : 0]; };
+                if constexpr (HD == 128)
+                    fma4(o, lane >> 5 ? of(1) : of(0), *dst);
+                else
+                    fma4(o, lane >> 5 ? (lane & 16 ? of(3) : of(2)) : (lane & 16 ? of(1) : of(0)), *dst);
+            }
+            *dst = o;
+        });
         flushed = true;
     };
 
@@ -1113,6 +1186,20 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
         // e, one 4x4x1 MFMA adds p[row][head i] * V[row][4*vj + e] for the
         // four heads of a quad (A: lane 4b+i gives p of head i for its row;
         // B: each lane its own V component).
+        // (With PART every probability is read ahead of the products: left in
+        // place, each set's read waited for in turn.  Graph replay, Llama-3-8B
+        // heads ctx 256 5.04 -> 4.88 us, 1000 5.78 -> 5.67; Llama-3.1-405B
+        // 13.9 -> 13.5.  Whole-pass launches measured 0-1% slower with it.)
+        float pa[GQ][VS];
+        if constexpr (MFMA && PART) {
+#pragma unroll
+            for (int q = 0; q < GQ; q++)
+#pragma unroll
+                for (int vs = 0; vs < VS; vs++) {
+                    const int h = 4 * q + (lane & 3);
+                    pa[q][vs] = (h < G) ? p_lds[wave][(vs * RPV + vg) * G + h] : 0.0f;
+                }
+        }
 #pragma unroll
         for (int vs = 0; vs < VS; vs++) {
             const int r = vs * RPV + vg;
@@ -1130,21 +1217,21 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
             for (int q = 0; q < GQ; q++) {
                 if constexpr (MFMA) {
                     const int h = 4 * q + (lane & 3);
-                    const float pa = (h < G) ? p_lds[wave][r * G + h] : 0.0f;
-                    acc[q][0] = __builtin_amdgcn_mfma_f32_4x4x1f32(pa, vb[vs].x, acc[q][0], 0, 0, 0);
-                    acc[q][1] = __builtin_amdgcn_mfma_f32_4x4x1f32(pa, vb[vs].y, acc[q][1], 0, 0, 0);
-                    acc[q][2] = __builtin_amdgcn_mfma_f32_4x4x1f32(pa, vb[vs].z, acc[q][2], 0, 0, 0);
-                    acc[q][3] = __builtin_amdgcn_mfma_f32_4x4x1f32(pa, vb[vs].w, acc[q][3], 0, 0, 0);
+                    const float p = PART ? pa[q][vs] : (h < G) ? p_lds[wave][r * G + h] : 0.0f;
+                    acc[q][0] = __builtin_amdgcn_mfma_f32_4x4x1f32(p, vb[vs].x, acc[q][0], 0, 0, 0);
+                    acc[q][1] = __builtin_amdgcn_mfma_f32_4x4x1f32(p, vb[vs].y, acc[q][1], 0, 0, 0);
+                    acc[q][2] = __builtin_amdgcn_mfma_f32_4x4x1f32(p, vb[vs].z, acc[q][2], 0, 0, 0);
+                    acc[q][3] = __builtin_amdgcn_mfma_f32_4x4x1f32(p, vb[vs].w, acc[q][3], 0, 0, 0);
                 } else {
                     // acc[q][e][i]: head 4q+i at dim 4*vj + e, as the MFMA leaves it
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
                         if (4 * q + i >= G) continue;
-                        const float pa = p_lds[wave][r * G + 4 * q + i];
-                        acc[q][0][i] += pa * vb[vs].x;
-                        acc[q][1][i] += pa * vb[vs].y;
-                        acc[q][2][i] += pa * vb[vs].z;
-                        acc[q][3][i] += pa * vb[vs].w;
+                        const float p = p_lds[wave][r * G + 4 * q + i];
+                        acc[q][0][i] += p * vb[vs].x;
+                        acc[q][1][i] += p * vb[vs].y;
+                        acc[q][2][i] += p * vb[vs].z;
+                        acc[q][3][i] += p * vb[vs].w;
                     }
                 }
             }
@@ -1229,14 +1316,16 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
         }
     }
 
-    // Per-wave partials to LDS: every V row slot its own accumulator.
+    // Per-wave partials to LDS.
     if constexpr (FLAT) {
         flush();
-    } else
+    } else if constexpr (!PART) {
 #pragma unroll
-    for (int h = 0; h < G; h++)
-        comb_o[wave][vg][h][vj] = make_float4(acc[h / 4][0][h % 4], acc[h / 4][1][h % 4],
-                                              acc[h / 4][2][h % 4], acc[h / 4][3][h % 4]);
+        for (int h = 0; h < G; h++)
+            comb_o[wave][vg][h][vj] = make_float4(acc[h / 4][0][h % 4], acc[h / 4][1][h % 4],
+                                                  acc[h / 4][2][h % 4], acc[h / 4][3][h % 4]);
+    } else
+        slot_sums<HD, G>(acc, lane, [&](int, int h, float4 o) { comb_o[wave][0][h][vj] = o; });
 #pragma unroll
     for (int h = 0; h < G; h++) {
         const float lw = score_rows_sum(l_run[h]);
@@ -1278,13 +1367,13 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
         // left to the compiler, two reads were in flight at a time between
         // the fused multiply-adds, one LDS round trip per wave's partial.
         float mw[NW], lw[NW];
-        float4 ow[NW][RPV];
+        float4 ow[NW][SLOTS];
 #pragma unroll
         for (int w = 0; w < NW; w++) mw[w] = comb_m[ch][w];
 #pragma unroll
         for (int w = 0; w < NW; w++)
 #pragma unroll
-            for (int r = 0; r < RPV; r++) ow[w][r] = comb_o[w][r][ch][cd4];
+            for (int r = 0; r < SLOTS; r++) ow[w][r] = comb_o[w][r][ch][cd4];
 #pragma unroll
         for (int w = 0; w < NW; w++) lw[w] = comb_l[ch][w];
         __builtin_amdgcn_sched_barrier(0);
@@ -1296,7 +1385,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
         for (int w = 0; w < NW; w++) {
             const float sc = (mw[w] == -INFINITY) ? 0.0f : fast_exp2(mw[w] - M);
 #pragma unroll
-            for (int r = 0; r < RPV; r++) fma4(o, sc, ow[w][r]);
+            for (int r = 0; r < SLOTS; r++) fma4(o, sc, ow[w][r]);
             L += sc * lw[w];
         }
         if (single) {
