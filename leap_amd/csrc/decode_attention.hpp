@@ -26,6 +26,9 @@
 //     of kSubGroup consecutive chunks fold into one record each, and the last
 //     sub-group to finish folds those.  No fold pulls more than about 80 KiB
 //     through one CU.
+// A batch whose groups do not cut evenly over the CUs runs the same body over
+// equal runs of rows that may end one sequence and begin the next (the flat
+// launches, decode_attention_flat_kernel).
 //
 // XCD placement.  Workgroups are dealt to the XCDs round-robin by workgroup
 // id, so id % 8 names the XCD (the same holds within a 1-, 2- or 4-XCD

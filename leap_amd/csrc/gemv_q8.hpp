@@ -3,10 +3,10 @@
 // float scale per group of gs consecutive values of a row, as
 // QuantizedTransformer::quantize (QuantizedTransformer.cpp:338-357) and
 // ::matmul (:359-652) compute them.
-//   - q8_gemv_kernel<..., kRms = true,  kResid = false>: xb = rmsnorm(x),
+//   - q8_gemv_kernel<..., kQ8InRms, false>: xb = rmsnorm(x),
 //     quantized per group, then q, k, v = the stacked int8 Wq/Wk/Wv . xb
 //     (QuantizedTransformer.cpp:664-678);
-//   - q8_gemv_kernel<..., kRms = false, kResid = true>: the attention output
+//   - q8_gemv_kernel<..., kQ8InF32, true>: the attention output
 //     quantized per group, then x += Wo . that (the wo matmul and the residual
 //     after the attention block).
 //
