@@ -855,11 +855,13 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     __shared__ float4 q_lds[G][HD / 4];  // rotated, scaled q of the group's heads
     // The waves' partial outputs, [wave][V row slot][head][column]; also staging
     // for the new token (per wave) and the merge's scratch.  With PART a wave
-    // sums its slots first (slot_sums): same process, graph replay, Llama-3-8B
-    // heads ctx 256 5.10 -> 4.95 us, TinyLlama ctx 64 3.56 -> 3.48, and in flat
-    // launches a quarter to half the bytes of every flush.  Whole-pass launches
-    // keep the slots apart: the sums' extra steps made Llama-3-8B ctx 4096
-    // 0.8% slower.
+    // sums its slots first (slot_sums), which in flat launches also halves (or
+    // quarters) the bytes of every flush.  With the probabilities read ahead
+    // (below), same process, back to back: Llama-3-8B heads ctx 256 5.07 ->
+    // 4.93 us, ctx 1000 5.84 -> 5.66, TinyLlama ctx 256 4.64 -> 4.56, ctx 1000
+    // 5.43 -> 5.25, Llama-3.1-405B ctx 4096 14.5 -> 14.1.  Whole-pass launches
+    // keep the slots apart: the same steps made Llama-3-8B ctx 4096 0.8%
+    // slower.
     constexpr int SLOTS = PART ? 1 : RPV;
     // (a float4 per lane and wave at least, for the staging and the merge)
     constexpr int CSLOTS = SLOTS * G * D4 < kWave ? (kWave + G * D4 - 1) / (G * D4) : SLOTS;
@@ -1190,7 +1192,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
         // four heads of a quad (A: lane 4b+i gives p of head i for its row;
         // B: each lane its own V component).
         // (With PART every probability is read ahead of the products: left in
-        // place, each set's read waited for in turn.  Graph replay, Llama-3-8B
+        // place, each set's read waited for in turn.  Back to back, Llama-3-8B
         // heads ctx 256 5.04 -> 4.88 us, 1000 5.78 -> 5.67; Llama-3.1-405B
         // 13.9 -> 13.5.  Whole-pass launches measured 0-1% slower with it.)
         float pa[GQ][VS];
