@@ -455,9 +455,17 @@ constexpr size_t kTlRingWords = (size_t)leap::kTlSlots * leap::kTlMaxWgs * leap:
 constexpr int kFlatPerCu = 2;
 constexpr long long kFlatOneBytes = 512ll << 20;
 bool equal_lengths(int n_seq, long long total_rows, int max_T) { return total_rows == (long long)n_seq * max_T; }
+// The flat kernel of a launch's view; nullptr where there is none: the twin
+// and quarter launch groups of small launches (launch_view), of which a handle
+// of more sequences can hold records enough, stay uniform launches.
+KernelFn flat_kernel(const LaunchShape &s)
+{
+    return s.head_dim == 64 ? pick_flat<64>(s.group, s.kv_split) : pick_flat<128>(s.group, s.kv_split);
+}
 int flat_launch(const LaunchShape &s, int n_seq, long long total_rows, int max_T)
 {
     const long long n_groups = (long long)n_seq * s.n_kv_heads;
+    if (!flat_kernel(s)) return 0;
     if (s.valu || s.split > 0 || s.max_flat < kFlatPerCu * s.n_cu / leap::kXcds) return 0;
     if (n_groups < 2 * leap::kXcds || n_groups > leap::kFlatMaxItems * leap::kXcds) return 0;
     const int cus = s.n_cu / leap::kXcds;
@@ -478,12 +486,43 @@ int flat_launch(const LaunchShape &s, int n_seq, long long total_rows, int max_T
     return s.group > 1 && total_rows * s.n_kv_heads >= (long long)min_run * kFlatPerCu * s.n_cu ? per_cu * cus : 0;
 }
 
+// The split-K workspace of a handle's launches: the most chunks per sequence
+// and workgroups per XCD of a flat launch that it serves, its records (each
+// a partial output and a (max, sum) pair) and its counter words.
+struct Workspace {
+    int max_chunks, max_flat;
+    size_t rows, counter_ints;
+};
+Workspace workspace_for(const leap_hip_attention_config &c, int n_cu)
+{
+    // launch groups (kv_view), their records and counters: for max_batch *
+    // n_kv_heads groups, or for kXcds part-groups when a launch spreads fewer
+    // groups over the XCDs
+    const KvView kvv = kv_view(c.n_heads / c.n_kv_heads, c.n_kv_heads);
+    Workspace w{};
+    w.max_chunks = max_chunks_for(c.seq_len, c.head_dim, kvv.group, kvv.n_kv_heads, n_cu, leap::kMaxChunks);
+    const size_t n_pg = std::max<size_t>((size_t)c.max_batch * kvv.n_kv_heads, leap::kXcds);
+    // (and a flat launch's: records per XCD for its workgroups and at most
+    // kFlatMaxItems groups)
+    const int items = (int)std::min<size_t>((n_pg + leap::kXcds - 1) / leap::kXcds, leap::kFlatMaxItems);
+    w.max_flat = items >= 2 ? kFlatPerCu * n_cu / leap::kXcds : 0;
+    w.rows = std::max(n_pg * kvv.group * leap::records_per_head(w.max_chunks),
+                      (size_t)leap::kXcds * kvv.group * leap::flat_records(w.max_flat, items));
+    // (launch_view's two groups of 2 or 4 q heads per cache head, or four of
+    // 2: up to 2 kXcds groups, whose records fit in those of kXcds groups of
+    // 4 or 8)
+    const bool twins = (kvv.group == 8 || kvv.group == 4) && kvv.kv_split == 0;
+    const size_t n_ctr = std::max<size_t>(n_pg, twins ? 2 * leap::kXcds : 0);
+    w.counter_ints = n_ctr * leap::counters_per_group(std::max(w.max_chunks, w.max_flat));
+    return w;
+}
+
 // Enqueue a flat launch of n_wg workgroups per XCD.
 hipError_t launch_flat(const LaunchShape &s, const LaunchBuffers &b, int n_wg, int n_seq, const int *pos_dev,
                        int max_pos, long long total_rows, const float *q, const float *k, const float *v, float *out,
                        hipStream_t stream)
 {
-    KernelFn fn = s.head_dim == 64 ? pick_flat<64>(s.group, s.kv_split) : pick_flat<128>(s.group, s.kv_split);
+    KernelFn fn = flat_kernel(s);
     if (!fn || s.n_kv_heads >= 65536) return hipErrorInvalidValue;
     leap::StepArgs a{};
     a.q = q;
@@ -947,29 +986,13 @@ int leap_hip_attention_create(const leap_hip_attention_config *cfg, leap_hip_att
     CREATE_TRY(hipMemcpyAsync(h->rope, packed.data(), packed.size() * sizeof(float),
                               hipMemcpyHostToDevice, h->stream));
 
-    // launch groups (kv_view), their records and counters: for max_batch *
-    // n_kv_heads groups, or for kXcds part-groups when a launch spreads fewer
-    // groups over the XCDs
-    const KvView kvv = kv_view(h->group, c.n_kv_heads);
-    h->max_chunks = max_chunks_for(c.seq_len, c.head_dim, kvv.group, kvv.n_kv_heads, h->n_cu, leap::kMaxChunks);
-    const size_t n_pg = std::max<size_t>((size_t)c.max_batch * kvv.n_kv_heads, leap::kXcds);
-    // (and a flat launch's: records per XCD for its workgroups and at most
-    // kFlatMaxItems groups)
-    const int items = (int)std::min<size_t>((n_pg + leap::kXcds - 1) / leap::kXcds, leap::kFlatMaxItems);
-    if (items >= 2) {
-        h->max_flat = kFlatPerCu * h->n_cu / leap::kXcds;
-        CREATE_TRY(load_flat_table(c.head_dim));
-    }
-    const size_t ws_rows = std::max(n_pg * kvv.group * leap::records_per_head(h->max_chunks),
-                                    (size_t)leap::kXcds * kvv.group * leap::flat_records(h->max_flat, items));
-    CREATE_TRY(hipMalloc(&h->ws_o, ws_rows * c.head_dim * sizeof(float)));
-    CREATE_TRY(hipMalloc(&h->ws_ml, ws_rows * sizeof(float2)));
-    // (launch_view's two groups of 2 or 4 q heads per cache head, or four of
-    // 2: up to 2 kXcds groups, whose records fit in those of kXcds groups of
-    // 4 or 8)
-    const bool twins = (kvv.group == 8 || kvv.group == 4) && kvv.kv_split == 0;
-    const size_t n_ctr = std::max<size_t>(n_pg, twins ? 2 * leap::kXcds : 0);
-    h->counter_bytes = n_ctr * leap::counters_per_group(std::max(h->max_chunks, h->max_flat)) * sizeof(int);
+    const Workspace w = workspace_for(c, h->n_cu);
+    h->max_chunks = w.max_chunks;
+    h->max_flat = w.max_flat;
+    if (h->max_flat > 0) CREATE_TRY(load_flat_table(c.head_dim));
+    CREATE_TRY(hipMalloc(&h->ws_o, w.rows * c.head_dim * sizeof(float)));
+    CREATE_TRY(hipMalloc(&h->ws_ml, w.rows * sizeof(float2)));
+    h->counter_bytes = w.counter_ints * sizeof(int);
     CREATE_TRY(hipMalloc(&h->ws_po, (size_t)leap::kXcds * h->group * c.head_dim * sizeof(float)));
     CREATE_TRY(hipMalloc(&h->ws_pml, (size_t)leap::kXcds * h->group * sizeof(float2)));
     CREATE_TRY(hipMalloc(&h->counters, h->counter_bytes));
