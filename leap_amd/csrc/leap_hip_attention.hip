@@ -174,7 +174,6 @@ struct LaunchShape {
     int max_flat = 0;      // workgroups per XCD of a flat launch that the buffers hold records and counters for
 };
 
-
 // The device buffers of one launch (one layer): the cache slabs of sequence
 // 0 at this layer and the distance between sequences, the RoPE table, and
 // the split-K workspace (records_per_head(grid) records per head and
@@ -436,18 +435,35 @@ constexpr size_t kTlRingWords = (size_t)leap::kTlSlots * leap::kTlMaxWgs * leap:
 //     Llama-3-8B heads, 12 sequences of 2000 rows 46.9 -> 37.3, 3 of 4000
 //     27.6 -> 21.9 (33 chunks on 32 CUs); 6 (15/16 used) of 4000 35.2 ->
 //     37.5; 24 (3/4) of 1000-8000 36.7 -> 40.5 to 234.6 -> 232.7; 70B heads,
-//     12 of 2000 49.9 -> 40.1, 24 of 8000 276 -> 253.
+//     12 of 2000 49.9 -> 40.1, 24 of 8000 276 -> 253; Llama-2-7B heads (one q
+//     head per KV head), 3 of 2000 45.6 -> 36.6, 10 of 1000 65.1 -> 60.1.
 //     TinyLlama's heads (8 per KV head at head_dim 64), where the uniform
 //     chunks run one workgroup per CU, are bound by their products and take
 //     two: 32 sequences of 1000 rows 22.1 -> 18.7, of 4000 65.4 -> 49.5, 16 of
 //     1000 14.1 -> 12.8 (with the runs cut at the sequences' ends), but 8 of
 //     1000 (62 rows a run) 10.1 -> 14.1.
-//   - Ragged lengths: flat once a run holds kFlatRun rows (a shorter one
-//     costs more in starts and records than the even cut saves: Llama-3-8B
-//     heads, 24 of 30-300 rows (62 a run) 12.1 -> 13.2, 16 of 100-1000 (137)
-//     23.2 -> 18.1; 70B heads, 8 of 100-1000 (69) 13.9 -> 14.8, 12 (103) 21.1
-//     -> 17.5).  With one q head per KV head the uniform chunks measured as
-//     fast (the mean of 29 batches -0.3%).
+//   - Ragged lengths: flat once a run holds 64 rows, or 96 with 8 q heads per
+//     KV head (a shorter one costs more in starts and records than the even
+//     cut saves: Llama-3-8B heads, 24 of 30-300 rows (62 a run) 12.1 -> 13.2,
+//     16 of 100-1000 (137) 23.2 -> 18.1; 70B heads, 8 of 100-1000 (69) 13.9 ->
+//     14.8, 12 (103) 21.1 -> 17.5).  With one q head per KV head the uniform
+//     chunks measured as fast (the mean of 29 batches -0.3%).
+//   - Lengths of at least 3/4 of the longest in the mean, equal ones too: the
+//     uniform launch cuts near-equal chunks, and flat has to make up for its
+//     starts.  Flat only while uniform_use, times what the starts add to the
+//     rows, is under a line: 9/10 (4/5 for equal lengths with up to 4 q heads
+//     per KV head; 3/4 where the two groups of a head of 16 q heads share its
+//     rows in L2, which the runs part).  Over 1900 batches of 2-64 sequences
+//     of 200-4000 rows of seven head shapes the lines leave 2.7% less time
+//     than flat launches for all, and 0.5% more than the better of the two for
+//     each.  Above a line, flat -> uniform: Llama-3-8B heads, 32 sequences of
+//     198-200 rows 16.2 -> 13.3, of 998-1000 46.4 -> 42.0, 8 of 4000 46.6 ->
+//     43.6; 70B heads, 28 equal ones of 500 26.4 -> 23.3; 128/8/128, 24 equal
+//     ones of 500 38.7 -> 32.1; 16/16/64, 20 equal ones of 200 11.8 -> 11.2.
+//     Below it, uniform -> flat: Llama-3-8B heads, 12 of 1998-2000 45.8 ->
+//     35.5, 48 of 1600-2000 125.5 -> 110.2.  TinyLlama's heads, bound by
+//     products (above), keep flat launches for every spread, and equal lengths
+//     up to a line of 1.05: 28 of 1000 18.0 -> 16.9, of 200 8.8 -> 10.6.
 // Two workgroups per CU, but one for 4 q heads per KV head or fewer from
 // kFlatOneBytes on: Llama-3-8B heads, 64 sequences of 400-4000 rows (1.2 GB)
 // 181.3 -> 175.2, 32 of 800-8000 177.9 -> 174.0; 12 of 400-4000 (210 MB)
@@ -455,6 +471,31 @@ constexpr size_t kTlRingWords = (size_t)leap::kTlSlots * leap::kTlMaxWgs * leap:
 constexpr int kFlatPerCu = 2;
 constexpr long long kFlatOneBytes = 512ll << 20;
 bool equal_lengths(int n_seq, long long total_rows, int max_T) { return total_rows == (long long)n_seq * max_T; }
+// The rows that a start counts as in a flat launch of n_wg workgroups per XCD
+// over `items` groups each: equal lengths that the runs divide are cut at the
+// sequences' ends when a start counts as none.
+int flat_start_rows(int n_wg, int items, int n_seq, long long total_rows, int max_T)
+{
+    return equal_lengths(n_seq, total_rows, max_T) && n_wg % items == 0 ? 0 : leap::kFlatSegmentRows;
+}
+// Items (groups) per XCD of a batch, at most.
+int flat_items(const LaunchShape &s, int n_seq)
+{
+    return (int)(((long long)n_seq * s.n_kv_heads + leap::kXcds - 1) / leap::kXcds);
+}
+// The share of the CUs' time that the uniform launch spends on the batch's
+// rows: its workgroups come in whole rounds over the CUs, and each takes its
+// chunk in whole passes.
+double uniform_use(const LaunchShape &s, int n_seq, long long total_rows, int max_T)
+{
+    const int cus = s.n_cu / leap::kXcds, items = flat_items(s, n_seq);
+    const int even = even_chunks_for(s, n_seq, total_rows, max_T);
+    const int chunk = even ? (max_T + even - 1) / even : choose_chunk(s, n_seq, total_rows, max_T);
+    const long long wgs = (long long)items * (even ? even : (max_T + chunk - 1) / chunk);
+    const long long rounds = (wgs + cus - 1) / cus;
+    const int rows = round_up(chunk, leap::rows_per_pass(s.head_dim, s.group, kWaves));
+    return (double)items * (double)total_rows / n_seq / ((double)rounds * cus * rows);
+}
 // The flat kernel of a launch's view; nullptr where there is none: the twin
 // and quarter launch groups of small launches (launch_view), of which a handle
 // of more sequences can hold records enough, stay uniform launches.
@@ -469,21 +510,29 @@ int flat_launch(const LaunchShape &s, int n_seq, long long total_rows, int max_T
     if (s.valu || s.split > 0 || s.max_flat < kFlatPerCu * s.n_cu / leap::kXcds) return 0;
     if (n_groups < 2 * leap::kXcds || n_groups > leap::kFlatMaxItems * leap::kXcds) return 0;
     const int cus = s.n_cu / leap::kXcds;
-    const int items = (int)((n_groups + leap::kXcds - 1) / leap::kXcds);
+    const int items = flat_items(s, n_seq);
     const long long bytes = total_rows * (long long)s.n_kv_heads * s.head_dim * 8ll;
-    const int per_cu = s.group <= 4 && bytes >= kFlatOneBytes ? 1 : kFlatPerCu;
-    if (equal_lengths(n_seq, total_rows, max_T)) {
-        if (s.group == 8 && s.head_dim == 64 && kFlatPerCu * cus % items == 0)
+    const int n_wg = cus * (s.group <= 4 && bytes >= kFlatOneBytes ? 1 : kFlatPerCu);
+    const bool equal = equal_lengths(n_seq, total_rows, max_T);
+    const bool products_bound = s.group == 8 && s.head_dim == 64;
+    if (total_rows * 4 >= 3ll * n_seq * max_T && (equal || !products_bound)) {
+        const double mean = (double)total_rows / n_seq;
+        const double starts = 1.0 + flat_start_rows(n_wg, items, n_seq, total_rows, max_T) / mean;
+        const double line = s.kv_split ? 0.75 : products_bound ? 1.05 : equal && s.group <= 4 ? 0.8 : 0.9;
+        if (uniform_use(s, n_seq, total_rows, max_T) * starts >= line) return 0;
+    }
+    if (equal) {
+        if (products_bound && kFlatPerCu * cus % items == 0)
             return (long long)max_T * items >= 120ll * kFlatPerCu * cus ? kFlatPerCu * cus : 0;
         const int even = even_chunks_for(s, n_seq, total_rows, max_T);
         const int chunk = choose_chunk(s, n_seq, total_rows, max_T);
         const long long wgs = (long long)items * (even ? even : (max_T + chunk - 1) / chunk);
         if (wgs < 3 * cus / 4) return 0;  // small: the launch leaves CUs out on purpose
         const long long rounds = (wgs + cus - 1) / cus;
-        return wgs * (s.group == 8 ? 10 : 4) < rounds * cus * (s.group == 8 ? 9 : 3) ? per_cu * cus : 0;
+        return wgs * (s.group == 8 ? 10 : 4) < rounds * cus * (s.group == 8 ? 9 : 3) ? n_wg : 0;
     }
     const int min_run = s.group == 8 ? 96 : 64;
-    return s.group > 1 && total_rows * s.n_kv_heads >= (long long)min_run * kFlatPerCu * s.n_cu ? per_cu * cus : 0;
+    return s.group > 1 && total_rows * s.n_kv_heads >= (long long)min_run * kFlatPerCu * s.n_cu ? n_wg : 0;
 }
 
 // The split-K workspace of a handle's launches: the most chunks per sequence
@@ -543,10 +592,7 @@ hipError_t launch_flat(const LaunchShape &s, const LaunchBuffers &b, int n_wg, i
     a.n_kv_heads = s.n_kv_heads;
     a.grid_chunks = n_wg;
     a.n_groups = n_seq * s.n_kv_heads;
-    // Equal lengths that the runs divide are cut at the sequences' ends when
-    // a start counts as no rows.
-    const int items = (a.n_groups + leap::kXcds - 1) / leap::kXcds;
-    a.chunk = equal_lengths(n_seq, total_rows, max_pos + 1) && n_wg % items == 0 ? 0 : leap::kFlatSegmentRows;
+    a.chunk = flat_start_rows(n_wg, flat_items(s, n_seq), n_seq, total_rows, max_pos + 1);
     a.scale_log2 = (float)(1.4426950408889634 / std::sqrt((double)s.head_dim));
     a.by_grid_chunks = leap::make_fastdiv((uint32_t)n_wg);
     a.by_kv_heads = leap::make_fastdiv((uint32_t)s.n_kv_heads);

@@ -1,6 +1,7 @@
 """The host's rules that route a launch: every call they send to a flat launch
-has a kernel and a workspace, on the CPU over many shapes and handles, and on
-the device for calls of a part of a handle's sequences."""
+has a kernel and a workspace, and batches on both sides of their lines take the
+route that measured faster, on the CPU over many shapes and handles; on the
+device, calls of a part of a handle's sequences."""
 import os
 import shutil
 import subprocess
