@@ -470,6 +470,7 @@ constexpr size_t kTlRingWords = (size_t)leap::kTlSlots * leap::kTlMaxWgs * leap:
 // 39.2 -> 41.2.
 constexpr int kFlatPerCu = 2;
 constexpr long long kFlatOneBytes = 512ll << 20;
+constexpr int kFlatMeanRows = 224;
 bool equal_lengths(int n_seq, long long total_rows, int max_T) { return total_rows == (long long)n_seq * max_T; }
 // The rows that a start counts as in a flat launch of n_wg workgroups per XCD
 // over `items` groups each: equal lengths that the runs divide are cut at the
@@ -531,7 +532,8 @@ int flat_launch(const LaunchShape &s, int n_seq, long long total_rows, int max_T
         const long long rounds = (wgs + cus - 1) / cus;
         return wgs * (s.group == 8 ? 10 : 4) < rounds * cus * (s.group == 8 ? 9 : 3) ? n_wg : 0;
     }
-    const int min_run = s.group == 8 ? 96 : 64;
+    const bool long_mean = total_rows >= (long long)kFlatMeanRows * n_seq;
+    const int min_run = s.group == 8 ? 96 : s.group == 4 && s.head_dim == 64 && long_mean ? 40 : 64;
     return s.group > 1 && total_rows * s.n_kv_heads >= (long long)min_run * kFlatPerCu * s.n_cu ? n_wg : 0;
 }
 

@@ -85,6 +85,9 @@ const struct {
     {64, 8, 128, 16, 2000, 16 * 1100, true},
     {32, 8, 128, 24, 300, 24 * 160, false},
     {32, 8, 128, 16, 2011, 0, true},
+    {32, 8, 64, 4, 2000, 3869, true},
+    {32, 8, 64, 8, 1000, 0, true},
+    {32, 8, 64, 48, 130, 48 * 80, false},
 };
 
 }  // namespace

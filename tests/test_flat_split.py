@@ -45,6 +45,7 @@ CASES = [
     (32, 8, 128, [1, 700, 63, 1200, 64, 65, 900, 1203]),
     (24, 8, 128, [1203, 1, 1, 700, 192, 900, 1200, 63]),
     (16, 8, 64, [700, 1200, 1300, 1, 900, 65]),
+    (32, 8, 64, [2000, 1, 900, 65]),                                # 46 rows a run
     (64, 8, 128, [2000, 1, 1500, 129, 1100, 700, 512, 400]),       # 8 q heads per KV head, two-level merges
     (32, 4, 64, [1500, 1, 1100] + [700 + 7 * i for i in range(13)]),  # four KV heads: an XCD has every other sequence
     (128, 8, 128, [2000, 1100]),                                    # 16 q heads per KV head (two launch groups)
