@@ -141,6 +141,20 @@ static_assert(alignof(Q8Args) == 8, "argument layout");
 #define LEAP_Q8_PRELOAD_PARAMS                                                                                  \
     const float *pre_x, const float *pre_rms_w, const int8_t *pre_w, const float *pre_ws, int pre_rows, int pre_per_wg
 
+// Float4 pairs (8 registers each) of the ordered chain that are read ahead, of
+// n4: all of them while they fit beside the rest, else the most that divide n4.
+// More than these spill: with 16 waves (128 registers) Llama-3-70B q/k/v 17.2
+// -> 20.6 us; at group size 32 with 8 waves (256) or 12 (168) all 32 or 24 took
+// 20-116 bytes of scratch (sub-block of 3072 with 24 KV heads 17.1 us, now 16.5;
+// of Llama-3-8B 17.6 either way).
+__host__ __device__ constexpr int q8_chain_unroll(int n4, int waves)
+{
+    const int most = waves >= 16 ? 8 : waves >= 12 ? 20 : 24;
+    int u = n4 < most ? n4 : most;
+    while (n4 % u) u--;
+    return u;
+}
+
 // What a kernel instance of (NL, L, J, NWV, WPR) is made of.
 template <int NL, int L, int J, int NWV, int WPR>
 struct Q8Shape {
@@ -299,9 +313,8 @@ __global__ __launch_bounds__(NWV * 64) void q8_gemv_kernel(LEAP_Q8_PRELOAD_PARAM
         const float4 *f4 = reinterpret_cast<const float4 *>(lds_f + tid * NGP);
         const float4 *c4 = reinterpret_cast<const float4 *>(lds_c + tid * NGP);
         // every LDS read ahead of the chain (0.05-0.3 us per launch against 4
-        // groups ahead); with 16 waves that would spill (Llama-3-70B q/k/v
-        // 17.2 -> 20.6 us)
-        constexpr int kChainUnroll = NWV >= 16 ? 8 : NG / 4;
+        // groups ahead) as far as the registers of a wave hold them
+        constexpr int kChainUnroll = q8_chain_unroll(NG / 4, NWV);
 #pragma unroll kChainUnroll
         for (int j = 0; j < NG / 4; j++) {
             const float4 f = f4[j], c = c4[j];
