@@ -471,6 +471,9 @@ constexpr size_t kTlRingWords = (size_t)leap::kTlSlots * leap::kTlMaxWgs * leap:
 constexpr int kFlatPerCu = 2;
 constexpr long long kFlatOneBytes = 512ll << 20;
 constexpr int kFlatMeanRows = 224;
+// The rows of a batch whose count the caller does not give: as if the lengths
+// were spread evenly up to the longest.
+long long rows_estimate(int n_seq, int max_T) { return (long long)n_seq * max_T / 2 + 1; }
 bool equal_lengths(int n_seq, long long total_rows, int max_T) { return total_rows == (long long)n_seq * max_T; }
 // The rows that a start counts as in a flat launch of n_wg workgroups per XCD
 // over `items` groups each: equal lengths that the runs divide are cut at the
@@ -1305,9 +1308,7 @@ int leap_hip_attention_step_batched_async(leap_hip_attention *h, int layer, int 
     if (total_rows < 0 || total_rows > (long long)n_seq * (max_pos + 1))
         return set_err(h, -EINVAL, "total_rows %lld outside [0, %lld]", total_rows,
                        (long long)n_seq * (max_pos + 1));
-    // Without the host's row count, size the chunks as if the lengths were
-    // spread evenly up to the longest.
-    const long long rows = total_rows > 0 ? total_rows : (long long)n_seq * (max_pos + 1) / 2 + 1;
+    const long long rows = total_rows > 0 ? total_rows : rows_estimate(n_seq, max_pos + 1);
     return launch(h, layer, n_seq, pos, 0, max_pos, rows, q, k_new, v_new, out,
                   (hipStream_t)stream);
 }

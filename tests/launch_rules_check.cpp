@@ -3,7 +3,11 @@
 // sequences, fewer sequences than the handle holds, and row counts given or
 // estimated, a flat launch's kernel exists and its records and counters fit
 // in the handle's workspace; and batches on both sides of the rule's lines take
-// the route that measured faster.  Built and run by tests/test_launch_rules.py.
+// the route that measured faster.  With "route" as its argument, it answers
+// calls read from its input instead: q heads, KV heads, head_dim, seq_len,
+// max_batch, sequences, the longest and all rows (0: not given) -> workgroups
+// per XCD of the flat launch, 0 for a uniform one.  Built and run by
+// tests/test_launch_rules.py.
 #include "checkpoint.cpp"
 #include "leap_hip_attention.hip"
 
@@ -92,10 +96,18 @@ const struct {
 
 }  // namespace
 
-int main()
+int main(int argc, char **)
 {
+    if (argc > 1) {
+        int nh, nkv, hd, seq_len, max_batch, n_seq, max_T;
+        long long rows;
+        while (std::scanf("%d %d %d %d %d %d %d %lld", &nh, &nkv, &hd, &seq_len, &max_batch, &n_seq, &max_T, &rows) == 8)
+            std::printf("%d\n", flat_workgroups(handle(nh, nkv, hd, seq_len, max_batch, 256), n_seq,
+                                                rows > 0 ? rows : rows_estimate(n_seq, max_T), max_T));
+        return 0;
+    }
     for (const auto &r : kRoutes) {
-        const long long rows = r.rows > 0 ? r.rows : (long long)r.n_seq * r.max_T / 2 + 1;
+        const long long rows = r.rows > 0 ? r.rows : rows_estimate(r.n_seq, r.max_T);
         const int n_wg = flat_workgroups(handle(r.n_heads, r.n_kv_heads, r.head_dim, r.max_T, r.n_seq, 256), r.n_seq, rows, r.max_T);
         REQUIRE((n_wg > 0) == r.flat, "heads %d/%d/%d, %d sequences, longest %d, rows %lld: %d workgroups per XCD", r.n_heads,
                 r.n_kv_heads, r.head_dim, r.n_seq, r.max_T, r.rows, n_wg);
@@ -114,7 +126,7 @@ int main()
                             for (int max_T : {1, 31, 64, 100, 500, 1000, 1024, 2011, 3000, 4095, 4096, 5000, 6143, 8192,
                                               12288, 16384, 24576, 32768})
                                 // estimated (total_rows 0), equal lengths, ragged ones, one long among short
-                                for (long long rows : {(long long)n_seq * max_T / 2 + 1, (long long)n_seq * max_T,
+                                for (long long rows : {rows_estimate(n_seq, max_T), (long long)n_seq * max_T,
                                                        (long long)n_seq * max_T * 5 / 6, (long long)max_T + n_seq - 1}) {
                                     calls++;
                                     const LaunchShape s = launch_view(shape_of(&h), n_seq, rows);

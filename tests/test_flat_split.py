@@ -1,8 +1,9 @@
 """Flat launches: a batch whose groups do not cut evenly over the CUs, its
 rows laid end to end and cut into equal runs (decode_attention_flat_kernel).
-The split is checked on the host; on the device the batches here take the
-flat launch by the host's rule, at the edges of its runs, segments and items,
-and meet the oracle (or, where it is slow, the uniform chunks of set_split)."""
+The split is checked on the host, and that the batches here take the flat
+launch by the host's rule, at the edges of its runs, segments and items; on the
+device they meet the oracle (or, where it is slow, the uniform chunks of
+set_split)."""
 import os
 import shutil
 import subprocess
@@ -11,6 +12,7 @@ import numpy as np
 import pytest
 
 from tests.helpers import assert_close, normal, rng_for
+from tests.test_launch_rules import flat_workgroups
 from oracle import oracle as O
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -47,9 +49,9 @@ CASES = [
     (16, 8, 64, [700, 1200, 1300, 1, 900, 65]),
     (32, 8, 64, [2000, 1, 900, 65]),                                # 46 rows a run
     (64, 8, 128, [2000, 1, 1500, 129, 1100, 700, 512, 400]),       # 8 q heads per KV head, two-level merges
-    (32, 4, 64, [1500, 1, 1100] + [700 + 7 * i for i in range(13)]),  # four KV heads: an XCD has every other sequence
-    (128, 8, 128, [2000, 1100]),                                    # 16 q heads per KV head (two launch groups)
-    (32, 8, 128, [30 + (37 * i) % 71 for i in range(64)]),          # 64 items per XCD, the most
+    (32, 4, 64, [1700, 1, 1300] + [700 + 7 * i for i in range(13)]),  # four KV heads: an XCD has every other sequence
+    (128, 8, 128, [2600, 1100]),                                    # 16 q heads per KV head (two launch groups)
+    (32, 8, 128, [40 + (37 * i) % 71 for i in range(64)]),          # 64 items per XCD, the most
     # equal lengths that do not divide the CUs
     (32, 8, 128, [1000] * 3),
     (8, 8, 128, [300] * 12),
@@ -58,6 +60,23 @@ CASES = [
     (32, 4, 64, [1920] * 8),
     (32, 4, 64, [241] * 64),
 ]
+
+
+LONG = (32, 8, 128, [20000, 17, 9000, 130])
+# a position that the launch cannot serve, by sequence
+BAD = (32, 8, 128, [900, 300, 1000, 700, 350, 950, 1000, 600])
+BAD_AT = {1: -1, 3: 5000, 6: 1001}
+
+
+# a captured launch whose positions move between replays, sized for an upper bound and without a row count
+MOVING = (32, 8, 128, 1600, 8, 6, 1600, 0)
+
+
+def test_the_batches_here_take_the_flat_launch():
+    calls = [(nh, nkv, hd, max(Ts) + 1, len(Ts), len(Ts), max(Ts), sum(Ts)) for nh, nkv, hd, Ts in CASES + [LONG]]
+    calls.append((32, 8, 128, 1200, 8, 8, 1001, sum(BAD[3])))
+    calls.append(MOVING)
+    assert all(n > 0 for n in flat_workgroups(calls)), list(zip(calls, flat_workgroups(calls)))
 
 
 @pytest.mark.gpu
@@ -87,7 +106,7 @@ def test_flat_batch_matches_uniform_chunks_at_long_contexts(hip_device):
     fp32 sums of the same products in another order: each within 6e-7 of 64
     bits in the 2-norm at these lengths, so within 1e-5 of the largest value
     of each other."""
-    nh, nkv, hd, Ts = 32, 8, 128, [20000, 17, 9000, 130]
+    nh, nkv, hd, Ts = LONG
     rng = rng_for(78, 1)
     att, _ = _filled(nh, nkv, hd, max(Ts), Ts, rng)
     with att:
@@ -105,9 +124,7 @@ def test_flat_batch_bad_positions_write_nan_rows(hip_device):
     """A position outside the launch: its output row reads NaN, its cache rows
     stay, and the other sequences' results do not change."""
     import torch
-    nh, nkv, hd = 32, 8, 128
-    Ts = [900, 800, 1000, 700, 850, 950, 1000, 600]
-    bad = {1: -1, 3: 5000, 6: 1001}
+    (nh, nkv, hd, Ts), bad = BAD, BAD_AT
     rng = rng_for(79, 1)
     att, rows = _filled(nh, nkv, hd, 1200, Ts, rng)
     with att:
@@ -131,3 +148,48 @@ def test_flat_batch_bad_positions_write_nan_rows(hip_device):
             orc.key_cache[0, :T - 1], orc.value_cache[0, :T - 1] = rows[s]
             want, _ = orc.step(0, T - 1, q[s], k[s], v[s])
             assert_close(out[s], want, what=f"sequence {s}")
+
+
+@pytest.mark.gpu
+def test_flat_launch_replays_at_moving_positions(hip_device):
+    """One captured flat launch, replayed as the sequences grow: every replay
+    gives the eager launch's output and cache rows at those positions."""
+    import torch
+    nh, nkv, hd, seq_len, max_batch, n, max_T, rows = MOVING
+    from leap_amd.attention import HipAttention
+    with HipAttention(nh, nkv, hd, seq_len, max_batch=max_batch) as att:
+        att.kv_fill_normal(31, 0.1)
+        g = torch.Generator(device="cuda").manual_seed(32)
+        q = torch.randn(n, nh * hd, device="cuda", generator=g)
+        k, v = (torch.randn(n, nkv * hd, device="cuda", generator=g) for _ in range(2))
+        out = torch.zeros(n, nh * hd, device="cuda")
+        pos = torch.tensor([0, 700, 63, 1300, 64, 900], dtype=torch.int32, device="cuda")
+
+        def step(stream):
+            att.step_batched_async(0, n, pos.data_ptr(), max_T - 1, q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                   out.data_ptr(), stream, total_rows=rows)
+
+        s = torch.cuda.Stream()
+        step(s.cuda_stream)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            step(torch.cuda.current_stream().cuda_stream)
+        for grow in (0, 1, 63, 130):
+            pos += grow
+            torch.cuda.synchronize()
+            step(s.cuda_stream)
+            torch.cuda.synchronize()
+            want, at = out.clone(), pos.tolist()
+            want_kv = [att.kv_download(i, 0, p, p + 1) for i, p in enumerate(at)]
+            for rep in range(2):
+                for i, p in enumerate(at):
+                    att.kv_upload(i, 0, p, np.zeros((1, nkv * hd), np.float32), np.zeros((1, nkv * hd), np.float32))
+                out.zero_()
+                torch.cuda.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(out, want), f"positions {at}, replay {rep}"
+                for (wk, wv), i, p in zip(want_kv, range(n), at):
+                    gk, gv = att.kv_download(i, 0, p, p + 1)
+                    assert np.array_equal(gk, wk) and np.array_equal(gv, wv), f"sequence {i}"

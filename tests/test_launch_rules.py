@@ -2,9 +2,12 @@
 has a kernel and a workspace, and batches on both sides of their lines take the
 route that measured faster, on the CPU over many shapes and handles; on the
 device, calls of a part of a handle's sequences."""
+import atexit
+import functools
 import os
 import shutil
 import subprocess
+import tempfile
 
 import numpy as np
 import pytest
@@ -15,20 +18,36 @@ from oracle import oracle as O
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def test_every_flat_launch_has_a_kernel_and_a_workspace(tmp_path):
+@functools.lru_cache(maxsize=None)
+def _program():
+    """The check program's path: the host side from its source, the kernel tables from the built library."""
     hipcc = "/opt/rocm/bin/hipcc" if os.path.exists("/opt/rocm/bin/hipcc") else shutil.which("hipcc")
     if not hipcc:
         pytest.skip("hipcc not found")
     from leap_amd.attention import load_library
     load_library()
     lib = os.path.join(ROOT, "leap_amd")
-    exe = tmp_path / "launch_rules_check"
-    # the program brings the host side from its source and takes the kernel tables from the built library
+    tmp = tempfile.mkdtemp()
+    atexit.register(shutil.rmtree, tmp, ignore_errors=True)
+    exe = os.path.join(tmp, "launch_rules_check")
     r = subprocess.run([hipcc, "-x", "hip", "--offload-arch=gfx950", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "leap_amd", "csrc"),
                         "-I", os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "launch_rules_check.cpp"),
-                        "-o", str(exe), "-L", lib, "-lleap_hip_attention", f"-Wl,-rpath,{lib}"], capture_output=True, text=True)
+                        "-o", exe, "-L", lib, "-lleap_hip_attention", f"-Wl,-rpath,{lib}"], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
-    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    return exe
+
+
+def flat_workgroups(calls):
+    """Workgroups per XCD of the flat launch of each call, 0 for a uniform one: calls are (q heads, KV heads,
+    head_dim, seq_len, max_batch, sequences, longest, all rows or 0)."""
+    r = subprocess.run([_program(), "route"], input="\n".join(" ".join(map(str, c)) for c in calls), capture_output=True,
+                       text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
+    return [int(x) for x in r.stdout.split()]
+
+
+def test_flat_launches_have_kernels_workspace_and_measured_lines():
+    r = subprocess.run([_program()], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
 
 
