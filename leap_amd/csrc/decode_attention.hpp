@@ -123,13 +123,18 @@ constexpr int kFlatSegmentRows = 128;
 constexpr int kFlatMinRun = 64;          // rows of a run at least: one pass of 4 waves
 constexpr int kFlatMaxItems = 64;        // items per XCD at most: one lane each
 // A run of a large batch holds thousands of rows.  Every kFlatFlushPasses
-// passes a wave adds its output accumulators to sums in LDS and starts them
-// anew, so that no fp32 sum is longer than a uniform chunk's.  Error against
-// 64 bits, 64 sequences of 512-8192 rows of Llama-3-8B's heads (runs of 8700):
-// 4.7e-7 without, 4.0e-7 at 16 passes, 3.6e-7 at 4 (uniform chunks of 768
-// rows: 3.8e-7); over seven batches of the three shapes the mean is 0.99 of
-// the uniform chunks'.  At 2 and 1 passes it is 0.98 and TinyLlama's batches
-// are 6-9% slower.
+// passes a wave adds its output accumulators to sums in LDS and its row sums
+// to a second register, and starts them anew: a sum over n passes is n / 4
+// additions of sums over 4, where a uniform chunk of a ragged batch is one
+// chain of about 12 passes (and one of a large equal batch, of up to all of
+// them).  Error against 64 bits, 64 sequences of 512-8192 rows of Llama-3-8B's
+// heads (runs of 8700 rows): 4.7e-7 without, 4.0e-7 at 16 passes, 3.6e-7 at 4
+// (uniform chunks of 768 rows: 3.8e-7); over seven batches of the three shapes
+// the mean is 0.99 of the uniform chunks'.  At 2 and 1 passes it is 0.98 and
+// TinyLlama's batches are 6-9% slower.  Equal scores, whose sum rounds the same
+// way at every addition (n 2^-26 at the worst), six sequences of 30000-90000
+// rows: 2.0e-6 with the row sums of a run in one chain, 7.8e-7 now (TinyLlama's
+// batches 0.7% slower for it, the others as fast).
 constexpr int kFlatFlushPasses = 4;
 
 // Segment (workgroup w, item i) has record w + i among its XCD's: along the
@@ -879,7 +884,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     // f < HD/32, so one load instruction reads 128 contiguous bytes of each of
     // eight rows.  MFMA block lane/4 = 8*kq + ksl multiplies four q heads
     // (A: lane 4*block + i gives head 4*quad + i) by its four rows (B) at one
-    // dim; the eight slices are summed afterwards (slice_sum).
+    // dim; the eight slices are summed afterwards (slice_sum2).
     const int kj = lane & 3, ksl = (lane >> 2) & 7, kq = lane >> 5;
     const int krow = 4 * kq + kj;
     const int srow = score_row(lane);  // the row whose score this lane holds
@@ -1017,15 +1022,17 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
         for (int e = 0; e < 4; e++) acc[q][e] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // FLAT: this wave's outputs so far, relative to 2^m_sum, as its partials in
-    // the combine buffer
-    float m_sum[FLAT ? G : 1];
+    // the combine buffer, and its sums of p
+    float m_sum[FLAT ? G : 1], l_sum[FLAT ? G : 1];
     bool flushed = false;
     auto flush = [&]() {
         float ratio[G];  // from the sums' reference max to the current one
 #pragma unroll
         for (int h = 0; h < G; h++) {
-            ratio[h] = fast_exp2(m_sum[h] - m_ref[h]);
+            ratio[h] = flushed ? fast_exp2(m_sum[h] - m_ref[h]) : 0.0f;
             m_sum[h] = m_ref[h];
+            l_sum[h] = flushed ? ratio[h] * l_sum[h] + l_run[h] : l_run[h];
+            l_run[h] = 0.0f;
         }
         slot_sums<HD, G>(acc, lane, [&](int h0, int h, float4 o) {
             float4 *dst = &comb_o[wave][0][h][vj];
@@ -1333,7 +1340,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
         slot_sums<HD, G>(acc, lane, [&](int, int h, float4 o) { comb_o[wave][0][h][vj] = o; });
 #pragma unroll
     for (int h = 0; h < G; h++) {
-        const float lw = score_rows_sum(l_run[h]);
+        const float lw = score_rows_sum(FLAT ? l_sum[h] : l_run[h]);
         if (lane == 0) {
             comb_l[h][wave] = lw;
             comb_m[h][wave] = m_ref[h];
