@@ -1395,7 +1395,8 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
         for (int w = 0; w < NW; w++) M = fmaxf(M, mw[w]);
 #pragma unroll
         for (int w = 0; w < NW; w++) {
-            const float sc = (mw[w] == -INFINITY) ? 0.0f : fast_exp2(mw[w] - M);
+            // (finite: the reference starts at kLowest and only grows)
+            const float sc = fast_exp2(mw[w] - M);
 #pragma unroll
             for (int r = 0; r < SLOTS; r++) fma4(o, sc, ow[w][r]);
             L += sc * lw[w];
