@@ -863,7 +863,7 @@ __device__ __forceinline__ void decode_attention_body(const StepArgs &args, cons
     // sums its slots first (slot_sums), which in flat launches also halves (or
     // quarters) the bytes of every flush.  With the probabilities read ahead
     // (below), same process, back to back: Llama-3-8B heads ctx 256 5.07 ->
-    // 4.93 us, ctx 1000 5.84 -> 5.66, TinyLlama ctx 256 4.64 -> 4.56, ctx 1000
+    // 4.93 us, ctx 1000 5.84 -> 5.66, TinyLlama ctx 256 within 2%, ctx 1000
     // 5.43 -> 5.25, Llama-3.1-405B ctx 4096 14.5 -> 14.1.  Whole-pass launches
     // keep the slots apart: the same steps made Llama-3-8B ctx 4096 0.8%
     // slower.

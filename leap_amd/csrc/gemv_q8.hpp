@@ -116,12 +116,12 @@ __device__ __forceinline__ float group_max_w(float v)
 // idled 64-96 of a team's 256 threads, and the rows per team came in steps
 // that left 1.2-1.5 rounds of workgroups at Llama-2's widths.  us per launch,
 // back to back over 1 GiB of weights, before -> now: Llama-3-8B q/k/v (6144 x
-// 4096) 7.29 -> 6.33, wo 5.44 -> 5.05 (the weights alone on the old grid 5.16
-// and 4.05); Llama-2-13B q/k/v (15360 x 5120) 24.4 -> 16.2, wo 9.3 -> 6.8;
-// Llama-2-7B q/k/v (12288 x 4096) 14.3 -> 10.7; Llama-3-70B q/k/v (10240 x
-// 8192) 18.8 -> 17.2, wo 14.2 -> 14.1; TinyLlama q/k/v (2560 x 2048) 4.14 ->
-// 2.95, wo 3.47 -> 2.96; Llama-3.2-3B q/k/v (5120 x 3072) 5.51 -> 5.11, wo
-// 4.40 -> 3.88.
+// 4096) 7.29 -> 6.33, wo 5.44 -> 5.05 (of the sub-block's 21.2 the bare streams
+// of its three grids take 16.2); Llama-2-13B q/k/v (15360 x 5120) 24.4 -> 16.2,
+// wo 9.3 -> 6.8; Llama-2-7B q/k/v (12288 x 4096) 14.3 -> 10.7; Llama-3-70B
+// q/k/v (10240 x 8192) 18.8 -> 17.2, wo 14.2 -> 14.1; TinyLlama q/k/v (2560 x
+// 2048) 4.14 -> 2.95, wo 3.47 -> 2.96; Llama-3.2-3B q/k/v (5120 x 3072) 5.51 ->
+// 5.11, wo 4.40 -> 3.88.
 //
 // Issue order: the input first, then the rows' scales and the weight rows
 // (96 KiB a workgroup for Wq/Wk/Wv at Llama-3-8B), all before anything waits.

@@ -21,7 +21,9 @@ struct Q8Entry {
 // 12 x 2 6.68, 6 x 4 6.78, 16 (teams of 2) x 3 7.01; 10 rows as 5 x 2 2.94,
 // 10 x 1 3.19; 60 rows as 12 x 5 16.5, 10 x 6 16.8, 6 x 10 21.8; 20 rows at
 // 5120 as 10 x 2 7.04, 5 x 4 7.49; 40 rows at 8192 as 16 waves in teams of 2
-// x 5 17.2, 8 x 5 17.8, 10 x 4 25.7.
+// x 5 17.2, 8 x 5 17.8, 10 x 4 25.7.  Rows per CU between two sizes leave slots
+// idle (5120 with 10 KV heads: 30 of 60), which still beats a team per row:
+// its sub-block 26.7 -> 24.3.
 #define LEAP_Q8_K(NL, L, J, NWV, WPR, K)                                                                \
     {NL, L, J * NWV / WPR, NWV * 64, K, leap::q8_gemv_kernel<NL, L, J, NWV, WPR, K, K != leap::kQ8InRms>, \
      leap::q8_floor_kernel<NL, L, J, NWV, WPR>},

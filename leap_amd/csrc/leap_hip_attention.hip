@@ -441,7 +441,9 @@ constexpr size_t kTlRingWords = (size_t)leap::kTlSlots * leap::kTlMaxWgs * leap:
 //     chunks run one workgroup per CU, are bound by their products and take
 //     two: 32 sequences of 1000 rows 22.1 -> 18.7, of 4000 65.4 -> 49.5, 16 of
 //     1000 14.1 -> 12.8 (with the runs cut at the sequences' ends), but 8 of
-//     1000 (62 rows a run) 10.1 -> 14.1.
+//     1000 (62 rows a run) 10.1 -> 14.1.  Since the packed scores, batches of
+//     4-64 at runs of 64-96 rows: flat 1-20% slower in each; at 104-128, 7%
+//     faster (32 sequences) to 8% slower (64); the line is 120.
 //   - Ragged lengths: flat once a run holds 64 rows, or 96 with 8 q heads per
 //     KV head (a shorter one costs more in starts and records than the even
 //     cut saves: Llama-3-8B heads, 24 of 30-300 rows (62 a run) 12.1 -> 13.2,
