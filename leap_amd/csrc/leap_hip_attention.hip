@@ -470,6 +470,12 @@ constexpr size_t kTlRingWords = (size_t)leap::kTlSlots * leap::kTlMaxWgs * leap:
 // kFlatOneBytes on: Llama-3-8B heads, 64 sequences of 400-4000 rows (1.2 GB)
 // 181.3 -> 175.2, 32 of 800-8000 177.9 -> 174.0; 12 of 400-4000 (210 MB)
 // 39.2 -> 41.2.
+// Row counts that the caller does not give are estimated as half the longest
+// each: ragged.  On the other side of kFlatOneBytes that costs up to 2%; equal
+// lengths gain or lose by it (Llama-3-8B heads, uniform -> flat, 16 of 1000
+// 28.5 -> 26.3, 12 of 1000 20.3 -> 21.6, 48 of 500 35.0 -> 37.9); the same calls
+// with lengths spread up to the longest take 20.7 -> 17.7, 17.4 -> 15.3 and 27.8
+// -> 24.3.
 constexpr int kFlatPerCu = 2;
 constexpr long long kFlatOneBytes = 512ll << 20;
 constexpr int kFlatMeanRows = 224;
