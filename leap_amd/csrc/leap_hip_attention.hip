@@ -450,6 +450,13 @@ constexpr size_t kTlRingWords = (size_t)leap::kTlSlots * leap::kTlMaxWgs * leap:
 //     16 of 100-1000 (137) 23.2 -> 18.1; 70B heads, 8 of 100-1000 (69) 13.9 ->
 //     14.8, 12 (103) 21.1 -> 17.5).  With one q head per KV head the uniform
 //     chunks measured as fast (the mean of 29 batches -0.3%).
+//     With 4 at head_dim 64 already from 40 rows, where the mean length is
+//     kFlatMeanRows: four uniform workgroups of these fit on a CU, and a grid
+//     of that many puts the chunks past the shorter sequences' ends on the same
+//     CUs.  32/8/64, sequences of a tenth of the longest and up, uniform ->
+//     flat: 4 to 2000 rows 11.9 -> 8.9, 8 to 1000 without the row count 11.7 ->
+//     9.0, 12 to 600 11.3 -> 9.2; below the mean, 48 to 130 9.6 -> 10.9, 16 of
+//     5-50 under a longest of 400 without the row count 5.2 -> 6.5.
 //   - Lengths of at least 3/4 of the longest in the mean, equal ones too: the
 //     uniform launch cuts near-equal chunks, and flat has to make up for its
 //     starts.  Flat only while uniform_use, times what the starts add to the
