@@ -30,9 +30,10 @@ def _program():
     tmp = tempfile.mkdtemp()
     atexit.register(shutil.rmtree, tmp, ignore_errors=True)
     exe = os.path.join(tmp, "launch_rules_check")
-    r = subprocess.run([hipcc, "-x", "hip", "--offload-arch=gfx950", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "leap_amd", "csrc"),
-                        "-I", os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "launch_rules_check.cpp"),
-                        "-o", exe, "-L", lib, "-lleap_hip_attention", f"-Wl,-rpath,{lib}"], capture_output=True, text=True)
+    r = subprocess.run([hipcc, "-x", "hip", "--offload-arch=gfx950", "-O2", "-std=c++17", "-Xclang", "-target-feature",
+                        "-Xclang", "-packed-fp32-ops", "-I", os.path.join(ROOT, "leap_amd", "csrc"), "-I",
+                        os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "launch_rules_check.cpp"), "-o", exe,
+                        "-L", lib, "-lleap_hip_attention", f"-Wl,-rpath,{lib}"], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
     return exe
 
